@@ -5,7 +5,9 @@ One step = one iclblasSgemm call (device-pointer mode, inputs resident in HBM)
 on the handle's stream; K steps are timed with HIP events recorded on that
 stream. Prints ONE JSON line:
   value        split-BF16 SGEMM throughput, useful TFLOP/s = 2 m n k / t
-  paths        both paths: TFLOP/s, fraction of their MFMA peak, max error vs FP64
+  paths        both paths and the FP32 math mode as selected (fp32_auto: the exact
+               three-way split on BF16 MFMA): TFLOP/s, fraction of their MFMA peak,
+               max error vs FP64
   roofline     the split-BF16 kernel: executed BF16 TFLOP/s (3 products) vs 2516.6
   roofline_fp32  the FP32-MFMA kernel vs 157.3
   cpu_baseline the reference's CPU GEMM (restated cpu_gemm, double accumulation,
@@ -30,6 +32,14 @@ sys.path.insert(0, str(ROOT))
 
 PEAK_FP32_MFMA = 157.3   # TFLOP/s, MI355X dense FP32 matrix
 PEAK_BF16_MFMA = 2516.6  # TFLOP/s, MI355X dense BF16 matrix (no sparsity)
+FP32_MFMA_KERNEL = "sgemm_f32_dma_256x256w8k32"  # the FP32-MFMA path of the headline line
+
+
+def executed(impl: str):
+    """(MFMA products per useful one, peak of their unit) of a GEMM implementation."""
+    if "split3" in impl:
+        return 6.0, PEAK_BF16_MFMA
+    return (3.0, PEAK_BF16_MFMA) if "bf16x3" in impl else (1.0, PEAK_FP32_MFMA)
 
 
 def parse():
@@ -40,7 +50,8 @@ def parse():
     ap.add_argument("--size", type=int, default=8192)
     ap.add_argument("--no-cpu-baseline", action="store_true")
     ap.add_argument("--cpu-seconds", type=float, default=12.0, help="target CPU-baseline sample duration")
-    ap.add_argument("--paths", default="fp32,bf16x3")
+    ap.add_argument("--paths", default="fp32,fp32_auto,bf16x3",
+                    help="fp32: the FP32-MFMA kernel by name; fp32_auto: the FP32 math mode as selected; bf16x3")
     ap.add_argument("--impl", default="", help="comma list, one implementation name per path (empty = automatic)")
     ap.add_argument("--trans", default="NN", help="NN, NT, TN or TT for the timed op")
     ap.add_argument("--no-check", action="store_true", help="skip the FP64 error check (profiling runs)")
@@ -566,10 +577,10 @@ def cgemm_rows(h, ib, stream, steps: int) -> dict:
             ms = _time(stream, lambda: ib.check(ib.iclblasCgemm(h.value, ta, 0, n, n, n, alpha, A.data_ptr(), n,
                                                                 B.data_ptr(), n, beta, Cw.data_ptr(), n)), steps, 2)
             tf = flops / (ms * 1e-3) / 1e12
+            times, peak = executed(h.last_implementation())
             res[path] = {"implementation": h.last_implementation(), "ms": ms, "tflops": tf,
                          "frac_of_fp32_mfma_peak": tf / PEAK_FP32_MFMA,
-                         "executed_frac_of_mfma_peak": (tf / PEAK_FP32_MFMA) if path == "fp32"
-                         else 3 * tf / PEAK_BF16_MFMA,
+                         "executed_frac_of_mfma_peak": times * tf / peak,
                          "max_abs_err": float(err.max()), "normwise_rel_err": float(err.norm() / ref.abs().norm()),
                          "max_err_over_bound_unit": ratio}
             del err, C, Cw
@@ -653,9 +664,10 @@ def sgemm_line(a, h, ib, stream, dev):
     results = {}
     impls = a.impl.split(",") if a.impl else []
     for pi, path in enumerate(a.paths.split(",")):
-        mode = ib.MATH_FP32 if path == "fp32" else ib.MATH_SPLIT_BF16X3
+        mode = ib.MATH_SPLIT_BF16X3 if path == "bf16x3" else ib.MATH_FP32
         h.set_math_mode(mode)
-        h.set_implementation(impls[pi] if pi < len(impls) else None)
+        by_path = FP32_MFMA_KERNEL if path == "fp32" else None
+        h.set_implementation(impls[pi] if pi < len(impls) else by_path)
 
         def step():
             ib.check(ib.iclblasSgemm(h.value, ta, tb, m, n, k, 1.0, tA.data_ptr(), n, tB.data_ptr(), n, 0.0,
@@ -684,14 +696,13 @@ def sgemm_line(a, h, ib, stream, dev):
         kern_ms = kern_total / kern_launches if kern_launches > 0 else None
         impl = h.last_implementation()
         tflops = flops / (ms * 1e-3) / 1e12
-        peak = PEAK_FP32_MFMA if path == "fp32" else PEAK_BF16_MFMA
-        per_launch = flops if path == "fp32" else 3.0 * flops  # executed MFMA flops of one launch
-        executed = per_launch / (kern_ms * 1e-3) / 1e12 if kern_ms else None
+        times, peak = executed(impl)
+        rate = times * flops / (kern_ms * 1e-3) / 1e12 if kern_ms else None  # executed MFMA flops
         results[path] = {"implementation": impl, "ms": ms, "tflops": tflops,
                          "frac_of_fp32_mfma_peak": tflops / PEAK_FP32_MFMA,
                          "kernel_ms": kern_ms, "kernel_launches": kern_launches,
-                         "executed_tflops": executed, "mfma_peak": peak,
-                         "mfma_frac": executed / peak if executed else None}
+                         "executed_tflops": rate, "mfma_peak": peak,
+                         "mfma_frac": rate / peak if rate else None}
         if C64 is not None:
             err = (tC.double() - C64).abs()
             ratio = float((err / (k * 2.0 ** -24 * absAB)).max())
@@ -705,7 +716,8 @@ def sgemm_line(a, h, ib, stream, dev):
         print(f"[bench] {path}: {ms:.3f} ms  {tflops:.1f} TFLOP/s  {results[path].get('max_err_over_bound_unit')}"
               f"  ({impl})", file=sys.stderr, flush=True)
 
-    head = "bf16x3" if "bf16x3" in results else "fp32"
+    h.set_implementation(None)
+    head = "bf16x3" if "bf16x3" in results else "fp32" if "fp32" in results else "fp32_auto"
     hr = results[head]
     # HBM bytes per launch come from the rocprofv3 FETCH_SIZE / WRITE_SIZE passes
     # summarised in profiles/sgemm_8192_hbm_traffic.md and recorded per kernel in

@@ -41,7 +41,8 @@ bool gemm_accept(const icl_gemm_variant& v, const GemmProblem& p)
     // The band flags of write_tri select tiles by whole 256 x 256 diagonal blocks.
     const bool band_ok = (p.args->write_tri & (ICL_TRI_OFF_BAND | ICL_TRI_BAND)) == 0 ||
                          (ICL_TRI_BAND_BLOCK % v.bm == 0 && ICL_TRI_BAND_BLOCK % v.bn == 0);
-    return v.kind == p.kind && v.math == p.math && (v.level3 || !level3_problem(*p.args)) && band_ok;
+    const bool ws_ok = v.math != ICL_MATH_FP32 || !v.workspace || p.optional_ws;
+    return v.kind == p.kind && v.math == p.math && (v.level3 || !level3_problem(*p.args)) && band_ok && ws_ok;
 }
 
 static bool aligned16(const void* p) { return (reinterpret_cast<uintptr_t>(p) & 15u) == 0; }
@@ -93,14 +94,33 @@ float gemm_score(const icl_gemm_variant& v, const GemmProblem& p)
         const double k0 = kTileOverheadK * v.bm * v.bn / (v.threads / 64);
         t_tile *= (double(g.K) + k0) / double(g.K) * 8192.0 / (8192.0 + k0);
     }
-    const double rounds = std::ceil(tiles / conc);
-    const double last = tiles - (rounds - 1.0) * conc;
-    double t = (rounds - 1.0) * t_tile + t_tile * std::max(last, kCUs) / conc;
-    if (rounds == 1.0) t *= 0.7 + 0.3 * std::min(tiles, kCUs) / kCUs;
-    if (gemm_needs_edge(v, p)) t *= 1.10;
-    if (v.workspace) t += (double(g.M) + double(g.N)) * double(g.K) * (p.kind == ICL_KIND_CGEMM ? 16.0 : 8.0) / 5e12;
+    auto grid_time = [&](double count, double at_once, double each) {
+        const double rounds = std::ceil(count / at_once);
+        const double last = count - (rounds - 1.0) * at_once;
+        double t = (rounds - 1.0) * each + each * std::max(last, kCUs) / at_once;
+        if (rounds == 1.0) t *= 0.7 + 0.3 * std::min(count, kCUs) / kCUs;
+        return t;
+    };
+    double t = grid_time(tiles, conc, t_tile);
+    if (v.workspace && v.math == ICL_MATH_FP32 && g.write_tri != ICL_TRI_NONE && g.M == g.N && v.bn == 256 &&
+        g.M >= 2 * ICL_TRI_BAND_BLOCK)
+        // runs off the diagonal blocks, then on them at a quarter of the tile, two per CU
+        t = grid_time(double(tri_tile_count(g.M, g.N, g.write_tri | ICL_TRI_OFF_BAND, v.bm, v.bn)), conc, t_tile) +
+            grid_time(double(tri_tile_count(g.M, g.N, g.write_tri | ICL_TRI_BAND, v.bm / 2, v.bn / 2)), 2 * kCUs,
+                      t_tile / 2);
+    if (gemm_needs_edge(v, p) && !(v.workspace && v.math == ICL_MATH_FP32)) t *= 1.10;
+    if (v.workspace && v.math == ICL_MATH_FP32) {
+        // three-way split: 4 read + 6 written bytes per real element, op(A) of a
+        // complex product expanded to two rows of two, and two more launches
+        const double a = p.kind == ICL_KIND_CGEMM ? 32.0 : 10.0, b = p.kind == ICL_KIND_CGEMM ? 20.0 : 10.0;
+        t += (a * double(g.M) + b * double(g.N)) * double(g.K) / 4.5e12 + 10e-6;
+    } else if (v.workspace) {
+        t += (double(g.M) + double(g.N)) * double(g.K) * (p.kind == ICL_KIND_CGEMM ? 16.0 : 8.0) / 5e12;
+    }
     return (float)(1.0 / t);
 }
+
+static const icl_gemm_variant* gemm_best(const GemmProblem& p);
 
 static bool forced_is_gemm_of_kind(const std::string& name, int kind)
 {
@@ -116,12 +136,37 @@ const icl_gemm_variant* gemm_select(iclblasContext* h, const GemmProblem& p)
     const bool level3 = level3_problem(*p.args);
     if (!h->forced_impl.empty() && forced_is_gemm_of_kind(h->forced_impl, p.kind)) {
         for (const icl_gemm_variant* v : gemm_registry())
-            if (h->forced_impl == v->name && (!level3 || v->level3)) return v;
+            if (h->forced_impl == v->name && (!level3 || v->level3) &&
+                (v->math != ICL_MATH_FP32 || !v->workspace || p.optional_ws))
+                return v;
     }
+    return gemm_best(p);
+}
+
+// The three-way split kernels are candidates from a packed depth of 256 (k, or 2 k
+// of a complex product) on: their error against float64 is 5% above FP32 MFMA's at
+// depth 65, 8% below it at 165 and 10 to 14% below it from 1000 on. Their workspace
+// (12 bytes per padded element of op(A) and op(B)^T at most) is bounded.
+// Below 1 GFLOP the pack and its launches take longer than the whole product.
+constexpr int kSplit3MinDepth = 256;
+constexpr double kSplit3MinMacs = 0.5e9; // real multiply-adds
+constexpr size_t kSplit3MaxBytes = size_t(8) << 30;
+static bool split3_candidate(int kind, const icl_gemm_args& g)
+{
+    const int c = kind == ICL_KIND_CGEMM ? 2 : 1;
+    return c * g.K >= kSplit3MinDepth && double(c) * c * g.M * double(g.N) * g.K >= kSplit3MinMacs;
+}
+
+// The accepted implementation with the highest score.
+static const icl_gemm_variant* gemm_best(const GemmProblem& p)
+{
     const icl_gemm_variant* best = nullptr;
     float best_score = -1.0f;
     for (const icl_gemm_variant* v : gemm_registry()) {
         if (!gemm_accept(*v, p)) continue;
+        if (v->math == ICL_MATH_FP32 && v->workspace &&
+            (!split3_candidate(p.kind, *p.args) || v->workspace(p.args) > kSplit3MaxBytes))
+            continue;
         const float s = gemm_score(*v, p);
         if (s > best_score) {
             best = v;
@@ -141,16 +186,61 @@ const icl_gemm_variant* gemm_select(iclblasContext* h, const GemmProblem& p)
 // 3 k 2^-24 |a||b| once k >= 256. Smaller K runs on FP32 MFMA instead.
 constexpr int kSplitMinK = 256;
 
+// Whether a product may use memory that only makes it faster: not when it could not
+// pay, when the caller has capped the handle's memory or forbidden allocation, and
+// not while the stream is being captured (a later call could free a workspace that
+// the graph would use).
+static bool optional_workspace(iclblasContext* h, int kind, const icl_gemm_args& g, hipStream_t s)
+{
+    if (g.K <= 0 || h->ext_ws || h->budget.limit || s != h->stream) return false;
+    if (h->forced_impl.empty() && !split3_candidate(kind, g)) return false;
+    hipStreamCaptureStatus capture = hipStreamCaptureStatusNone;
+    hip_check(hipStreamIsCapturing(s, &capture), "hipStreamIsCapturing");
+    return capture == hipStreamCaptureStatusNone;
+}
+
+// The product on a three-way split kernel `v`, then the FP32 MFMA kernel `native`
+// guarded by its range check. False when the workspace cannot be had.
+static bool run_split3(iclblasContext* h, const icl_gemm_variant* v, const icl_gemm_variant* native,
+                       const GemmProblem& p, hipStream_t s)
+{
+    icl_gemm_args g = *p.args;
+    void* ws = h->scratch[iclblasContext::kSlotSplit3].try_get(v->workspace(&g), s);
+    icl::DeviceScratch& word = h->scratch[iclblasContext::kSlotGuard];
+    const bool fresh = h->guard_epoch == 0;
+    g.guard = ws ? static_cast<unsigned long long*>(word.try_get(256, s)) : nullptr;
+    if (!g.guard) return false;
+    if (fresh)
+        hip_check(icl_axpby_2d(64, 1, 0.0f, nullptr, 0, 0.0f, reinterpret_cast<float*>(g.guard), 64, s), "axpby");
+    g.guard_epoch = ++h->guard_epoch;
+    hip_check(v->launch(&g, p.opa, p.opb, 0, ws, s), v->name);
+    GemmProblem q = p;
+    q.args = &g;
+    hip_check(native->launch(&g, p.opa, p.opb, gemm_needs_edge(*native, q) ? 1 : 0, nullptr, s), native->name);
+    return true;
+}
+
 // `stream`: the stream to run on (default the handle's; a variant with a
 // workspace always runs on the handle's stream).
 static void run_gemm(iclblasContext* h, int kind, int math, int opa, int opb, const icl_gemm_args& g, bool record,
                      hipStream_t stream = nullptr)
 {
     if (math == ICL_MATH_BF16X3 && g.K < kSplitMinK) math = ICL_MATH_FP32;
+    const hipStream_t s = stream ? stream : h->stream;
     GemmProblem p{kind, math, opa, opb, &g};
+    p.optional_ws = math == ICL_MATH_FP32 && optional_workspace(h, kind, g, s);
     const icl_gemm_variant* v = gemm_select(h, p);
     if (level3_problem(g) && !v->level3)
         throw status_error(ICLBLAS_STATUS_INTERNAL_ERROR, "level-3 GEMM options on a kernel without them");
+    if (v->math == ICL_MATH_FP32 && v->workspace) {
+        p.optional_ws = false;
+        const icl_gemm_variant* native = gemm_best(p);
+        if (run_split3(h, v, native, p, s)) {
+            if (record) h->last_impl = v->name;
+            return;
+        }
+        v = native;
+    }
     const bool edge = gemm_needs_edge(*v, p);
     void* ws = nullptr;
     if (v->workspace) {
@@ -167,9 +257,8 @@ static void run_gemm(iclblasContext* h, int kind, int math, int opa, int opb, co
     // and may run half of the prepass on the handle's side stream: offered for
     // products of at least 1024 tiles of that variant, never to a call that must
     // not allocate (the stream and its events are created on first use).
-    if (v->workspace && stream && stream != h->stream)
+    if (v->workspace && s != h->stream)
         throw status_error(ICLBLAS_STATUS_INTERNAL_ERROR, "GEMM with a workspace off the handle's stream");
-    const hipStream_t s = stream ? stream : h->stream;
     if (!v->workspace) hip_check(icl_timer_mark(s), "icl_timer_mark");
     const long tiles = (long)((g.M + v->bm - 1) / v->bm) * ((g.N + v->bn - 1) / v->bn);
     struct SideGuard {
@@ -252,6 +341,11 @@ static bool band_split_pays(iclblasContext* h, int kind, int math, int opa, int 
     if (!h->forced_impl.empty() || math != ICL_MATH_FP32 || g.kband != ICL_KBAND_NONE || g.M != g.N ||
         g.M < 2 * ICL_TRI_BAND_BLOCK || (g.write_tri != ICL_TRI_LOWER && g.write_tri != ICL_TRI_UPPER))
         return false;
+    {
+        GemmProblem whole{kind, math, opa, opb, &g};
+        whole.optional_ws = optional_workspace(h, kind, g, h->stream);
+        if (gemm_select(h, whole)->workspace) return false;
+    }
     auto est = [&](int tri) {
         icl_gemm_args t = g;
         t.write_tri = tri;

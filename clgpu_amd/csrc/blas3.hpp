@@ -16,6 +16,7 @@ struct GemmProblem {
     int math; // ICL_MATH_*
     int opa, opb;
     const icl_gemm_args* args;
+    bool optional_ws = false; // FP32 implementations that need a workspace are candidates
 };
 
 // Every registered GEMM implementation, in registration order.

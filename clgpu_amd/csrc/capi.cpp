@@ -82,6 +82,7 @@ ICLBLAS_API iclblasStatus_t iclblasCreate(iclblasHandle_t* handle)
     }
     h->own_stream = true;
     for (auto& s : h->scratch) s.set_budget(&h->budget);
+    h->budget.optional = &h->scratch[iclblasContext::kSlotSplit3];
     // The implementation name is copied on every call: room for the longest one
     // now, so that calls do not allocate host memory for it.
     h->last_impl.reserve(64);

@@ -96,6 +96,8 @@ __device__ __forceinline__ void c32dma_frag(const float* S, int rb, int q2, int 
 template <bool A_KC, bool CA, bool B_KC, bool CB, bool L3>
 __global__ void __launch_bounds__(C32DmaCfg::NT, 2) cgemm_f32_dma_kernel(GemmArgs g)
 {
+    if constexpr (L3)
+        if (guarded_off(g)) return;
     using Cfg = C32DmaCfg;
     extern __shared__ __attribute__((aligned(1024))) unsigned char lds_c32dma[];
     const int tid = threadIdx.x, lane = tid & 63;

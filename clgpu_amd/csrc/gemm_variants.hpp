@@ -14,11 +14,11 @@ struct VariantRegistrar {
 };
 
 // ---- SGEMM, FP32 MFMA ------------------------------------------------------
-// Problems that use the level-3 fields of icl_gemm_args run the kernel
-// instantiation that reads them; plain GEMMs run one compiled without them.
+// Problems that use the level-3 fields of icl_gemm_args, or a guard word, run the
+// kernel instantiation that reads them; plain GEMMs run one compiled without them.
 inline bool uses_level3(const GemmArgs* g)
 {
-    return g->write_tri != ICL_TRI_NONE || g->kband != ICL_KBAND_NONE || g->cflags != 0;
+    return g->guard != nullptr || g->write_tri != ICL_TRI_NONE || g->kband != ICL_KBAND_NONE || g->cflags != 0;
 }
 
 template <int TA, int TB, int BM, int BN, int BK, int WVM, int WVN, bool EDGE>

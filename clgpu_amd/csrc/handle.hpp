@@ -37,9 +37,11 @@ inline void hip_check(hipError_t e, const char* what)
 
 // Device memory held by a handle's scratch buffers, and its cap
 // (iclblasSetScratchLimit; 0 = none).
+class DeviceScratch;
 struct ScratchBudget {
     size_t limit = 0;
     size_t held = 0;
+    DeviceScratch* optional = nullptr; // given up when another buffer cannot be had
 };
 
 // A grow-only device allocation owned by the handle.
@@ -66,9 +68,36 @@ public:
             hip_check(hipStreamSynchronize(stream), "hipStreamSynchronize");
             release();
         }
-        hip_check(hipMalloc(&ptr_, want), "hipMalloc");
+        hipError_t e = hipMalloc(&ptr_, want);
+        if (e != hipSuccess && budget_ && budget_->optional && budget_->optional != this && budget_->optional->ptr_) {
+            (void)hipGetLastError();
+            hip_check(hipStreamSynchronize(stream), "hipStreamSynchronize");
+            budget_->optional->release();
+            e = hipMalloc(&ptr_, want);
+        }
+        if (e != hipSuccess) ptr_ = nullptr;
+        hip_check(e, "hipMalloc");
         cap_ = want;
         if (budget_) budget_->held += want;
+        return ptr_;
+    }
+
+    // The same for memory that only makes a call faster: nullptr instead of an
+    // error when the device has none left.
+    void* try_get(size_t bytes, hipStream_t stream)
+    {
+        if (bytes <= cap_ && ptr_) return ptr_;
+        if (ptr_) {
+            hip_check(hipStreamSynchronize(stream), "hipStreamSynchronize");
+            release();
+        }
+        if (hipMalloc(&ptr_, bytes) != hipSuccess) {
+            (void)hipGetLastError();
+            ptr_ = nullptr;
+            return nullptr;
+        }
+        cap_ = bytes;
+        if (budget_) budget_->held += bytes;
         return ptr_;
     }
 
@@ -237,13 +266,15 @@ extern thread_local const icl_side_lane* t_side_lane;
 
 struct iclblasContext {
     static constexpr int kTag = 0xB1A5;
-    static constexpr int kScratchSlots = 12;
+    static constexpr int kScratchSlots = 14;
     static constexpr int kSlotTrsmWorkspace = 6; // inverted diagonal blocks + solution of blocked STRSM
     static constexpr int kSlotGemmWorkspace = 7; // packed operands of split-BF16 GEMMs
     static constexpr int kSlotExpanded = 8;      // dense copy of a triangular / symmetric operand (level 3)
     static constexpr int kSlotLevel3Out = 9;     // TRMM result when C overlaps B in device memory mode
     static constexpr int kSlotGemvPartial = 10;  // split partial sums of GEMV
     static constexpr int kSlotRefine = 11;       // per-block maxima of the refinement convergence test
+    static constexpr int kSlotSplit3 = 12;       // packed operands of three-way split products (optional memory)
+    static constexpr int kSlotGuard = 13;        // guard word of those products
 
     int tag = kTag;
     int device = 0;
@@ -268,6 +299,9 @@ struct iclblasContext {
     // GEMM needing more than ext_ws_bytes fails with INVALID_VALUE.
     void* ext_ws = nullptr;
     size_t ext_ws_bytes = 0;
+    // Epoch of the last product that used the guard word (icl_gemm_args.guard); the
+    // word starts at 0 and never holds an epoch that has not been handed out.
+    unsigned long long guard_epoch = 0;
 
     static bool valid(const iclblasContext* h) { return h != nullptr && h->tag == kTag; }
 };

@@ -28,6 +28,12 @@ typedef struct icl_gemm_args {
     int write_tri; /* ICL_TRI_*: store only this triangle of C, leave the rest untouched */
     int kband;     /* ICL_KBAND_*: per-tile k window of a zero-padded triangular operand */
     int cflags;    /* ICL_CFLAG_*: complex epilogue options */
+    /* Guard word of a product that a kernel with a restricted operand range tries
+     * first (NULL: none). Its prepass stores guard_epoch into *guard when an operand
+     * lies outside the range; the kernel then leaves C alone, and the FP32 MFMA
+     * kernel launched after it with the same fields runs only in that case. */
+    unsigned long long* guard;
+    unsigned long long guard_epoch;
 } icl_gemm_args;
 
 enum {

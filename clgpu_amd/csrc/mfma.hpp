@@ -110,6 +110,10 @@ template <int BM, int BN>
 __device__ __forceinline__ bool tile_coords_level3(int write_tri, int kband, int tiles_m, int tiles_n, int& tm,
                                                    int& tn)
 {
+    if (write_tri == 0 && kband == 0) { // cflags or a guard only
+        tile_coords<8>(tiles_m, tiles_n, tm, tn);
+        return true;
+    }
     const int nb = gridDim.x;
     int b = blockIdx.x;
     if (write_tri != 0) {

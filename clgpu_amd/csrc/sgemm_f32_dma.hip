@@ -107,6 +107,8 @@ __device__ __forceinline__ void f32dma_frag(const float* S, int rb, int q2, int 
 template <int BM, int BN, int WVM, int WVN, bool A_KC, bool B_KC, bool L3, int BK = 16>
 __global__ void __launch_bounds__(WVM* WVN * 64) sgemm_f32_dma_kernel(GemmArgs g)
 {
+    if constexpr (L3)
+        if (guarded_off(g)) return;
     using Cfg = F32DmaCfg<BM, BN, WVM, WVN, BK>;
     extern __shared__ __attribute__((aligned(1024))) unsigned char lds_f32dma[];
     const int tid = threadIdx.x, lane = tid & 63;

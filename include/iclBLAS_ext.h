@@ -11,7 +11,12 @@
  *    handle's HIP stream and returns without waiting. Scalars (alpha, beta)
  *    are host pointers in both modes.
  *  - Math mode: ICLBLAS_MATH_FP32 runs SGEMM/CGEMM and the level-3 routines on
- *    FP32 MFMA. ICLBLAS_MATH_SPLIT_BF16X3 splits every FP32 operand x into
+ *    FP32 MFMA, or, for large products on a handle without a scratch cap and
+ *    outside stream capture, on BF16 MFMA with every operand split exactly into
+ *    three BF16 numbers (six products, FP32 accumulation): no bit of an operand
+ *    is lost and the error is below FP32 MFMA's. Operands with elements that do
+ *    not split exactly (infinities, NaN, magnitudes of 2^50 and more or below
+ *    2^-110) take FP32 MFMA. ICLBLAS_MATH_SPLIT_BF16X3 splits every FP32 operand x into
  *    hi = bf16(x), lo = bf16(x - hi) and forms hi*hi + hi*lo + lo*hi on BF16
  *    MFMA with FP32 accumulation, for products at least 256 deep (shallower
  *    ones stay on FP32 MFMA); the error stays within the FP32 bound
@@ -129,7 +134,7 @@ ICLBLAS_API iclblasStatus_t iclblasGetKernelTiming(iclblasHandle_t handle, float
  * scratch that stages host matrices in the host-pointer mode and holds the
  * workspaces: packed split-BF16 operands, TRSM and refinement temporaries,
  * level-3 expansions, GEMV partial sums), in bytes; 0 (the default) removes
- * the cap. A call that would grow them beyond it returns
+ * the cap. Under a cap the FP32 math mode keeps to kernels without workspaces. A call that would grow them beyond it returns
  * ICLBLAS_STATUS_ALLOC_FAILED, as when the device runs out of memory; buffers
  * already held are kept. Lowering the cap frees nothing. */
 ICLBLAS_API iclblasStatus_t iclblasSetScratchLimit(iclblasHandle_t handle, size_t bytes);
@@ -141,8 +146,8 @@ ICLBLAS_API iclblasStatus_t iclblasGetScratchUsage(iclblasHandle_t handle, size_
 
 /* SGEMM that allocates no memory. No counterpart in the reference: it is for
  * callers that cannot allocate (code under HIP graph capture, tight serving
- * loops, harnesses that forbid hipMalloc). Same arguments, validation and
- * result as iclblasSgemm, except that A, B and C are always device pointers
+ * loops, harnesses that forbid hipMalloc). Same arguments and validation
+ * as iclblasSgemm and a result within the same error bound, except that A, B and C are always device pointers
  * (whatever the memory mode) and the call is queued on the handle's stream and
  * returns without waiting. It calls no hipMalloc, hipFree or other allocating
  * routine: in the split-BF16 math mode the packed operands go to a device
@@ -150,8 +155,9 @@ ICLBLAS_API iclblasStatus_t iclblasGetScratchUsage(iclblasHandle_t handle, size_
  * from its first iclblasCreate there until the process ends. A call whose
  * packed operands need more than that, (M + N) * K * 4 bytes with M and N
  * rounded up to the kernel tile (256) and K to 32, returns
- * ICLBLAS_STATUS_INVALID_VALUE and queues nothing; the FP32 math mode and
- * products shallower than 256 use no scratch and have no such limit.
+ * ICLBLAS_STATUS_INVALID_VALUE and queues nothing; the FP32 math mode (always on
+ * FP32 MFMA here) and products shallower than 256 use no scratch and have no
+ * such limit.
  * ICLBLAS_STATUS_NOT_INITIALIZED: the scratch could not be set up on the
  * handle's GPU. Every call on one GPU shares that GPU's array: calls that
  * overlap on one GPU (other streams, other handles) race and must be ordered
