@@ -69,8 +69,8 @@ bool gemm_needs_edge(const icl_gemm_variant& v, const GemmProblem& p)
 // its tiles faster than a full chip does (a higher clock at the lower power,
 // less contention for L2 and HBM): (0.7 + 0.3 f) of that time, fitted to SSYRK
 // and CHERK triangles of 72 to 156 tiles. Variants with a pack prepass add its
-// HBM time ((M + N) * K elements at 4 read + 4 written bytes, twice that
-// complex, at 5 TB/s). The bounds-checked instantiation is taken to run 10%
+// HBM time ((M + N) * K elements at 4 read + 2 written bytes per plane, op(A) of
+// a complex product written twice, at 5 TB/s). The bounds-checked instantiation is taken to run 10%
 // slower.
 // For K <= 512 a tile's fixed cost (pipeline fill, C read and write) is no
 // longer small against its K loop: it is counted as kTileOverheadK * (elements
@@ -110,12 +110,13 @@ float gemm_score(const icl_gemm_variant& v, const GemmProblem& p)
                       t_tile / 2);
     if (gemm_needs_edge(v, p) && !(v.workspace && v.math == ICL_MATH_FP32)) t *= 1.10;
     if (v.workspace && v.math == ICL_MATH_FP32) {
-        // three-way split: 4 read + 6 written bytes per real element, op(A) of a
+        // three planes: 4 read + 6 written bytes per real element, op(A) of a
         // complex product expanded to two rows of two, and two more launches
         const double a = p.kind == ICL_KIND_CGEMM ? 32.0 : 10.0, b = p.kind == ICL_KIND_CGEMM ? 20.0 : 10.0;
         t += (a * double(g.M) + b * double(g.N)) * double(g.K) / 4.5e12 + 10e-6;
     } else if (v.workspace) {
-        t += (double(g.M) + double(g.N)) * double(g.K) * (p.kind == ICL_KIND_CGEMM ? 16.0 : 8.0) / 5e12;
+        const double a = p.kind == ICL_KIND_CGEMM ? 24.0 : 8.0, b = p.kind == ICL_KIND_CGEMM ? 16.0 : 8.0;
+        t += (a * double(g.M) + b * double(g.N)) * double(g.K) / 5e12;
     }
     return (float)(1.0 / t);
 }
