@@ -68,10 +68,13 @@ bool gemm_needs_edge(const icl_gemm_variant& v, const GemmProblem& p)
 // that fills only a fraction f of the CUs from the start (a single round) runs
 // its tiles faster than a full chip does (a higher clock at the lower power,
 // less contention for L2 and HBM): (0.7 + 0.3 f) of that time, fitted to SSYRK
-// and CHERK triangles of 72 to 156 tiles. Variants with a pack prepass add its
-// HBM time ((M + N) * K elements at 4 read + 2 written bytes per plane, op(A) of
-// a complex product written twice, at 5 TB/s). The bounds-checked instantiation is taken to run 10%
-// slower.
+// and CHERK triangles of 72 to 156 tiles. The bounds-checked instantiation runs at
+// 0.55 of the rate (FP32, 64 x 64 tiles: 53 of 100 TFLOP/s real, 71 of 131 complex), a
+// triangle's tiles at 0.8 (SSYRK 2048). Three-plane variants estimate their time
+// themselves. Split-BF16 variants with a prepass add its HBM time ((M + N) * K elements
+// at 4 read and 4 written bytes (8 and 8) at 5 TB/s);
+// whether a split-BF16 product needs a workspace, which a handle's cap may refuse, hangs
+// on these figures, which stay as they are.
 // For K <= 512 a tile's fixed cost (pipeline fill, C read and write) is no
 // longer small against its K loop: it is counted as kTileOverheadK * (elements
 // of C per wave) extra steps of K, normalised so that the rate at K = 8192 is
@@ -81,6 +84,7 @@ constexpr double kTileOverheadK = 0.12;
 float gemm_score(const icl_gemm_variant& v, const GemmProblem& p)
 {
     const icl_gemm_args& g = *p.args;
+    if (v.estimate && v.math == ICL_MATH_FP32) return (float)(1.0 / v.estimate(&g));
     constexpr double kCUs = 256.0;
     const double macs = p.kind == ICL_KIND_CGEMM ? 4.0 : 1.0; // real MACs per element MAC
     const double conc = kCUs * (v.occupancy > 0 ? v.occupancy : 1);
@@ -94,29 +98,16 @@ float gemm_score(const icl_gemm_variant& v, const GemmProblem& p)
         const double k0 = kTileOverheadK * v.bm * v.bn / (v.threads / 64);
         t_tile *= (double(g.K) + k0) / double(g.K) * 8192.0 / (8192.0 + k0);
     }
-    auto grid_time = [&](double count, double at_once, double each) {
-        const double rounds = std::ceil(count / at_once);
-        const double last = count - (rounds - 1.0) * at_once;
-        double t = (rounds - 1.0) * each + each * std::max(last, kCUs) / at_once;
-        if (rounds == 1.0) t *= 0.7 + 0.3 * std::min(count, kCUs) / kCUs;
-        return t;
-    };
-    double t = grid_time(tiles, conc, t_tile);
-    if (v.workspace && v.math == ICL_MATH_FP32 && g.write_tri != ICL_TRI_NONE && g.M == g.N && v.bn == 256 &&
-        g.M >= 2 * ICL_TRI_BAND_BLOCK)
-        // runs off the diagonal blocks, then on them at a quarter of the tile, two per CU
-        t = grid_time(double(tri_tile_count(g.M, g.N, g.write_tri | ICL_TRI_OFF_BAND, v.bm, v.bn)), conc, t_tile) +
-            grid_time(double(tri_tile_count(g.M, g.N, g.write_tri | ICL_TRI_BAND, v.bm / 2, v.bn / 2)), 2 * kCUs,
-                      t_tile / 2);
-    if (gemm_needs_edge(v, p) && !(v.workspace && v.math == ICL_MATH_FP32)) t *= 1.10;
-    if (v.workspace && v.math == ICL_MATH_FP32) {
-        // three planes: 4 read + 6 written bytes per real element, op(A) of a
-        // complex product expanded to two rows of two, and two more launches
-        const double a = p.kind == ICL_KIND_CGEMM ? 32.0 : 10.0, b = p.kind == ICL_KIND_CGEMM ? 20.0 : 10.0;
-        t += (a * double(g.M) + b * double(g.N)) * double(g.K) / 4.5e12 + 10e-6;
-    } else if (v.workspace) {
-        const double a = p.kind == ICL_KIND_CGEMM ? 24.0 : 8.0, b = p.kind == ICL_KIND_CGEMM ? 16.0 : 8.0;
-        t += (a * double(g.M) + b * double(g.N)) * double(g.K) / 5e12;
+    const double rounds = std::ceil(tiles / conc);
+    const double last = tiles - (rounds - 1.0) * conc;
+    double t = (rounds - 1.0) * t_tile + t_tile * std::max(last, kCUs) / conc;
+    if (rounds == 1.0) t *= 0.7 + 0.3 * std::min(tiles, kCUs) / kCUs;
+    if (v.math == ICL_MATH_FP32) {
+        if (gemm_needs_edge(v, p)) t *= 1.8;
+        if (g.write_tri != ICL_TRI_NONE) t *= 1.25;
+    } else {
+        if (gemm_needs_edge(v, p)) t *= 1.10;
+        if (v.workspace) t += (double(g.M) + double(g.N)) * double(g.K) * (p.kind == ICL_KIND_CGEMM ? 16.0 : 8.0) / 5e12;
     }
     return (float)(1.0 / t);
 }
@@ -145,17 +136,19 @@ const icl_gemm_variant* gemm_select(iclblasContext* h, const GemmProblem& p)
 }
 
 // The three-way split kernels are candidates from a packed depth of 256 (k, or 2 k
-// of a complex product) on: their error against float64 is 5% above FP32 MFMA's at
-// depth 65, 8% below it at 165 and 10 to 14% below it from 1000 on. Their workspace
-// (12 bytes per padded element of op(A) and op(B)^T at most) is bounded.
-// Below 1 GFLOP the pack and its launches take longer than the whole product.
+// of a complex product) on. Real products of up to 2 G multiply-adds stay on FP32
+// MFMA, so that iclblasSgemmNoAlloc, which has no workspace for the split, gives
+// iclblasSgemm's bits there (1024 x 1536 x 1024, 1.6 G: 46 us against about 40);
+// smaller complex ones than 0.5 G real multiply-adds take longer to pack than to
+// multiply. The workspace (12 bytes per padded element of op(A) and op(B)^T at most,
+// and 256 MiB of partial sums) is bounded.
 constexpr int kSplit3MinDepth = 256;
-constexpr double kSplit3MinMacs = 0.5e9; // real multiply-adds
+constexpr double kSplit3MinMacs[2] = {2e9, 0.5e9}; // real multiply-adds of a real, a complex product
 constexpr size_t kSplit3MaxBytes = size_t(8) << 30;
 static bool split3_candidate(int kind, const icl_gemm_args& g)
 {
     const int c = kind == ICL_KIND_CGEMM ? 2 : 1;
-    return c * g.K >= kSplit3MinDepth && double(c) * c * g.M * double(g.N) * g.K >= kSplit3MinMacs;
+    return c * g.K >= kSplit3MinDepth && double(c) * c * g.M * double(g.N) * g.K >= kSplit3MinMacs[c - 1];
 }
 
 // The accepted implementation with the highest score.
@@ -164,7 +157,7 @@ static const icl_gemm_variant* gemm_best(const GemmProblem& p)
     const icl_gemm_variant* best = nullptr;
     float best_score = -1.0f;
     for (const icl_gemm_variant* v : gemm_registry()) {
-        if (!gemm_accept(*v, p)) continue;
+        if (!gemm_accept(*v, p) || (p.no_ws && v->workspace)) continue;
         if (v->math == ICL_MATH_FP32 && v->workspace &&
             (!split3_candidate(p.kind, *p.args) || v->workspace(p.args) > kSplit3MaxBytes))
             continue;
@@ -175,7 +168,42 @@ static const icl_gemm_variant* gemm_best(const GemmProblem& p)
         }
     }
     if (!best) throw status_error(ICLBLAS_STATUS_NOT_SUPPORTED, "no GEMM implementation accepts the parameters");
+    if (best->math != ICL_MATH_FP32 && best->workspace) { // of the packed ones, the one that estimates the shortest time
+        double best_time = best->estimate(p.args);
+        for (const icl_gemm_variant* v : gemm_registry()) {
+            if (v == best || !v->workspace || !gemm_accept(*v, p)) continue;
+            const double t = v->estimate(p.args);
+            if (t < best_time) {
+                best = v;
+                best_time = t;
+            }
+        }
+    }
     return best;
+}
+
+// The packed operands of a split-BF16 product, 4 bytes per element (complex: 8), rounded up to whole 128-row tiles of 32-deep slabs.
+static size_t packed_bytes(int kind, const icl_gemm_args& g)
+{
+    auto up = [](int x, int m) { return (size_t)((x + m - 1) / m) * m; };
+    return (up(g.M, 128) + up(g.N, 128)) * up(g.K, 32) * (kind == ICL_KIND_CGEMM ? 8 : 4);
+}
+
+// A split-BF16 product on a handle with a cap: no partial sums, then the packed
+// implementation that needs the least. A complex one, whose op(A) is packed twice, runs
+// unpacked where the cap admits the operands packed once.
+static const icl_gemm_variant* capped_variant(iclblasContext* h, const icl_gemm_variant* v, GemmProblem& p,
+                                              icl_gemm_args& g)
+{
+    const icl::DeviceScratch& scratch = h->scratch[iclblasContext::kSlotGemmWorkspace];
+    g.whole_depth = 1;
+    if (scratch.fits(v->workspace(&g))) return v;
+    if (h->forced_impl.empty())
+        for (const icl_gemm_variant* u : gemm_registry())
+            if (u->workspace && gemm_accept(*u, p) && u->workspace(&g) < v->workspace(&g)) v = u;
+    if (scratch.fits(v->workspace(&g)) || p.kind != ICL_KIND_CGEMM || !scratch.fits(packed_bytes(p.kind, g))) return v;
+    p.no_ws = true;
+    return gemm_best(p);
 }
 
 // ---------------------------------------------------------------------------
@@ -223,7 +251,7 @@ static bool run_split3(iclblasContext* h, const icl_gemm_variant* v, const icl_g
 
 // `stream`: the stream to run on (default the handle's; a variant with a
 // workspace always runs on the handle's stream).
-static void run_gemm(iclblasContext* h, int kind, int math, int opa, int opb, const icl_gemm_args& g, bool record,
+static void run_gemm(iclblasContext* h, int kind, int math, int opa, int opb, icl_gemm_args g, bool record,
                      hipStream_t stream = nullptr)
 {
     if (math == ICL_MATH_BF16X3 && g.K < kSplitMinK) math = ICL_MATH_FP32;
@@ -242,9 +270,11 @@ static void run_gemm(iclblasContext* h, int kind, int math, int opa, int opb, co
         }
         v = native;
     }
+    if (v->workspace && h->budget.limit && !h->ext_ws) v = capped_variant(h, v, p, g);
     const bool edge = gemm_needs_edge(*v, p);
     void* ws = nullptr;
     if (v->workspace) {
+        if (h->ext_ws && v->workspace(&g) > h->ext_ws_bytes) g.whole_depth = 1;
         const size_t bytes = v->workspace(&g);
         if (bytes && h->ext_ws) {
             if (bytes > h->ext_ws_bytes)

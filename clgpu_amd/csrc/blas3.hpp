@@ -17,6 +17,7 @@ struct GemmProblem {
     int opa, opb;
     const icl_gemm_args* args;
     bool optional_ws = false; // FP32 implementations that need a workspace are candidates
+    bool no_ws = false;       // no implementation that needs a workspace is one
 };
 
 // Every registered GEMM implementation, in registration order.

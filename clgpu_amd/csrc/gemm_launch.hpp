@@ -4,12 +4,17 @@
 
 namespace icl {
 
-// Launches `kern(arg)` over ceil(M/BM) * ceil(N/BN) workgroups (M, N from g),
-// or over the tiles that meet the written triangle when g->write_tri is set.
-// Kernels that need more than 64 KiB of LDS get the dynamic-LDS limit raised
-// once per instantiation.
-template <int BM, int BN, int NT, size_t LDS, typename Kern, typename Arg>
-inline hipError_t launch_gemm(Kern kern, const GemmArgs* g, hipStream_t s, const Arg& arg)
+// Tiles of C that a launch covers.
+inline long gemm_tiles(const GemmArgs* g, int bm, int bn)
+{
+    return g->write_tri != ICL_TRI_NONE ? tri_tile_count(g->M, g->N, g->write_tri, bm, bn)
+                                        : (long)((g->M + bm - 1) / bm) * ((g->N + bn - 1) / bn);
+}
+
+// Launches `kern(arg)` over `blocks` workgroups of NT threads. Kernels that need more
+// than 64 KiB of LDS get the dynamic-LDS limit raised once per instantiation.
+template <int NT, size_t LDS, typename Kern, typename Arg>
+inline hipError_t launch_blocks(Kern kern, long blocks, hipStream_t s, const Arg& arg)
 {
     if constexpr (LDS > 65536) {
         static const hipError_t attr =
@@ -17,12 +22,17 @@ inline hipError_t launch_gemm(Kern kern, const GemmArgs* g, hipStream_t s, const
                                 static_cast<int>(LDS));
         if (attr != hipSuccess) return attr;
     }
-    const long tiles = g->write_tri != ICL_TRI_NONE ? tri_tile_count(g->M, g->N, g->write_tri, BM, BN)
-                                                    : (long)((g->M + BM - 1) / BM) * ((g->N + BN - 1) / BN);
-    if (tiles <= 0) return hipSuccess;
-    if (tiles > 0x7fffffffL) return hipErrorInvalidValue;
-    hipLaunchKernelGGL(kern, dim3((unsigned)tiles), dim3(NT), LDS, s, arg);
+    if (blocks <= 0) return hipSuccess;
+    if (blocks > 0x7fffffffL) return hipErrorInvalidValue;
+    hipLaunchKernelGGL(kern, dim3((unsigned)blocks), dim3(NT), LDS, s, arg);
     return hipGetLastError();
+}
+
+// Launches `kern(arg)` over the tiles of C.
+template <int BM, int BN, int NT, size_t LDS, typename Kern, typename Arg>
+inline hipError_t launch_gemm(Kern kern, const GemmArgs* g, hipStream_t s, const Arg& arg)
+{
+    return launch_blocks<NT, LDS>(kern, gemm_tiles(g, BM, BN), s, arg);
 }
 
 template <int BM, int BN, int NT, size_t LDS, typename Kern>

@@ -54,6 +54,13 @@ public:
 
     void set_budget(ScratchBudget* b) { budget_ = b; }
 
+    // Whether get(bytes) stays within the handle's cap.
+    bool fits(size_t bytes) const
+    {
+        const size_t want = bytes < 256 ? 256 : bytes;
+        return (ptr_ && bytes <= cap_) || !budget_ || !budget_->limit || budget_->held - cap_ + want <= budget_->limit;
+    }
+
     // Returns at least `bytes` of device memory. Growing waits for `stream` first
     // because queued work may still use the old allocation. Growing beyond the
     // handle's cap fails like an exhausted device (ALLOC_FAILED), before anything
@@ -62,7 +69,7 @@ public:
     {
         if (bytes <= cap_ && ptr_) return ptr_;
         const size_t want = bytes < 256 ? 256 : bytes;
-        if (budget_ && budget_->limit && budget_->held - cap_ + want > budget_->limit)
+        if (!fits(bytes))
             throw status_error(ICLBLAS_STATUS_ALLOC_FAILED, "scratch limit of the handle");
         if (ptr_) {
             hip_check(hipStreamSynchronize(stream), "hipStreamSynchronize");

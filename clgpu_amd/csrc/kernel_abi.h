@@ -34,6 +34,7 @@ typedef struct icl_gemm_args {
      * kernel launched after it with the same fields runs only in that case. */
     unsigned long long* guard;
     unsigned long long guard_epoch;
+    int whole_depth; /* nonzero: no split of the depth over workgroups (less workspace) */
 } icl_gemm_args;
 
 enum {
@@ -92,6 +93,8 @@ typedef struct icl_gemm_variant {
                           on a full MI355X (m = n = k = 8192, NN) */
     int occupancy;     /* workgroups resident per CU */
     int level3;        /* implements the level-3 fields write_tri, kband, cflags */
+    double (*estimate)(const icl_gemm_args* args); /* seconds a call takes, prepass included (NULL: the
+                                                      host's model of the fields above) */
 } icl_gemm_variant;
 
 /* Kernel timing hook. When the calling thread's handle has kernel timing on,

@@ -75,18 +75,20 @@ __device__ __forceinline__ bf16x8 bf16x8_neg(bf16x8 v)
     return __builtin_bit_cast(bf16x8, u);
 }
 
-// Maps blockIdx.x to a (tile_m, tile_n) pair.
-// 1) The dispatcher hands consecutive workgroup ids to the 8 XCDs round-robin,
-//    and each XCD has a private L2. Renumbering id -> (id % 8) * (n / 8) + id / 8
-//    gives every XCD a contiguous range of logical ids.
-// 2) Logical ids are rastered in groups of GROUP tile-rows so that workgroups
-//    running together on one XCD share A row-panels and B column-panels in L2.
-template <int GROUP>
-__device__ __forceinline__ void tile_coords(int tiles_m, int tiles_n, int& tm, int& tn)
+// Workgroup id -> logical id: the dispatcher hands consecutive workgroup ids to the 8
+// XCDs round-robin, and each XCD has a private L2. Renumbering
+// id -> (id % 8) * (n / 8) + id / 8 gives every XCD a contiguous range of logical ids.
+__device__ __forceinline__ int xcd_id(int b, int nb)
 {
-    const int nb = gridDim.x;
-    int b = blockIdx.x;
-    if ((nb & 7) == 0) b = (b & 7) * (nb >> 3) + (b >> 3);
+    return (nb & 7) == 0 ? (b & 7) * (nb >> 3) + (b >> 3) : b;
+}
+__device__ __forceinline__ int xcd_id() { return xcd_id(blockIdx.x, gridDim.x); }
+
+// Logical id -> tile: rastered in groups of GROUP tile-rows so that workgroups running
+// together on one XCD share A row-panels and B column-panels in L2.
+template <int GROUP>
+__device__ __forceinline__ void tile_raster(int b, int tiles_m, int tiles_n, int& tm, int& tn)
+{
     const int per_group = GROUP * tiles_n;
     const int g = b / per_group;
     const int first = g * GROUP;
@@ -94,6 +96,13 @@ __device__ __forceinline__ void tile_coords(int tiles_m, int tiles_n, int& tm, i
     const int r = b - g * per_group;
     tm = first + r % gsz;
     tn = r / gsz;
+}
+
+// Maps blockIdx.x to a (tile_m, tile_n) pair.
+template <int GROUP>
+__device__ __forceinline__ void tile_coords(int tiles_m, int tiles_n, int& tm, int& tn)
+{
+    tile_raster<GROUP>(xcd_id(), tiles_m, tiles_n, tm, tn);
 }
 
 // Tile numbering of the level-3 launches (the grid holds only the tiles that
@@ -105,19 +114,16 @@ __device__ __forceinline__ void tile_coords(int tiles_m, int tiles_n, int& tm, i
 //  - kband: all tiles, longest k window first, so that the round-robin
 //    dispatch over the XCDs spreads the long and the short tiles evenly and
 //    the short ones fill the tail.
-// Returns false (the workgroup has no tile) only for ids beyond that count.
+// Returns false (the workgroup has no tile) only for ids beyond that count. b: the
+// workgroup's logical id (kband without a triangle: its plain one).
 template <int BM, int BN>
-__device__ __forceinline__ bool tile_coords_level3(int write_tri, int kband, int tiles_m, int tiles_n, int& tm,
-                                                   int& tn)
+__device__ __forceinline__ bool tile_level3(int b, int write_tri, int kband, int tiles_m, int tiles_n, int& tm, int& tn)
 {
-    if (write_tri == 0 && kband == 0) { // cflags or a guard only
-        tile_coords<8>(tiles_m, tiles_n, tm, tn);
+    if (write_tri == 0 && kband == 0) { // a plain problem, cflags or a guard only
+        tile_raster<8>(b, tiles_m, tiles_n, tm, tn);
         return true;
     }
-    const int nb = gridDim.x;
-    int b = blockIdx.x;
     if (write_tri != 0) {
-        if ((nb & 7) == 0) b = (b & 7) * (nb >> 3) + (b >> 3);
         for (int i = 0; i < tiles_m; ++i) {
             int lo, cnt;
             tri_tile_row(write_tri, i, tiles_n, BM, BN, lo, cnt);
@@ -141,6 +147,14 @@ __device__ __forceinline__ bool tile_coords_level3(int write_tri, int kband, int
     tm = m_idx;
     tn = n_idx;
     return true;
+}
+
+template <int BM, int BN>
+__device__ __forceinline__ bool tile_coords_level3(int write_tri, int kband, int tiles_m, int tiles_n, int& tm,
+                                                   int& tn)
+{
+    return tile_level3<BM, BN>(write_tri == 0 && kband != 0 ? (int)blockIdx.x : xcd_id(), write_tri, kband, tiles_m,
+                               tiles_n, tm, tn);
 }
 
 } // namespace icl
