@@ -68,13 +68,12 @@ bool gemm_needs_edge(const icl_gemm_variant& v, const GemmProblem& p)
 // that fills only a fraction f of the CUs from the start (a single round) runs
 // its tiles faster than a full chip does (a higher clock at the lower power,
 // less contention for L2 and HBM): (0.7 + 0.3 f) of that time, fitted to SSYRK
-// and CHERK triangles of 72 to 156 tiles. The bounds-checked instantiation runs at
-// 0.55 of the rate (FP32, 64 x 64 tiles: 53 of 100 TFLOP/s real, 71 of 131 complex), a
-// triangle's tiles at 0.8 (SSYRK 2048). Three-plane variants estimate their time
-// themselves. Split-BF16 variants with a prepass add its HBM time ((M + N) * K elements
-// at 4 read and 4 written bytes (8 and 8) at 5 TB/s);
-// whether a split-BF16 product needs a workspace, which a handle's cap may refuse, hangs
-// on these figures, which stay as they are.
+// and CHERK triangles of 72 to 156 tiles. Variants with a pack prepass add its
+// HBM time ((M + N) * K elements at 4 read and 4 written bytes, complex 8 and 8, at
+// 5 TB/s). The bounds-checked instantiation is taken to run 10% slower: this ranks
+// implementations of one kind; whether a split-BF16 product needs a workspace, which a
+// handle's cap may refuse, hangs on these figures too. FP32 products on the three-way
+// split kernels are chosen by split_pays.
 // For K <= 512 a tile's fixed cost (pipeline fill, C read and write) is no
 // longer small against its K loop: it is counted as kTileOverheadK * (elements
 // of C per wave) extra steps of K, normalised so that the rate at K = 8192 is
@@ -84,7 +83,6 @@ constexpr double kTileOverheadK = 0.12;
 float gemm_score(const icl_gemm_variant& v, const GemmProblem& p)
 {
     const icl_gemm_args& g = *p.args;
-    if (v.estimate && v.math == ICL_MATH_FP32) return (float)(1.0 / v.estimate(&g));
     constexpr double kCUs = 256.0;
     const double macs = p.kind == ICL_KIND_CGEMM ? 4.0 : 1.0; // real MACs per element MAC
     const double conc = kCUs * (v.occupancy > 0 ? v.occupancy : 1);
@@ -102,13 +100,8 @@ float gemm_score(const icl_gemm_variant& v, const GemmProblem& p)
     const double last = tiles - (rounds - 1.0) * conc;
     double t = (rounds - 1.0) * t_tile + t_tile * std::max(last, kCUs) / conc;
     if (rounds == 1.0) t *= 0.7 + 0.3 * std::min(tiles, kCUs) / kCUs;
-    if (v.math == ICL_MATH_FP32) {
-        if (gemm_needs_edge(v, p)) t *= 1.8;
-        if (g.write_tri != ICL_TRI_NONE) t *= 1.25;
-    } else {
-        if (gemm_needs_edge(v, p)) t *= 1.10;
-        if (v.workspace) t += (double(g.M) + double(g.N)) * double(g.K) * (p.kind == ICL_KIND_CGEMM ? 16.0 : 8.0) / 5e12;
-    }
+    if (gemm_needs_edge(v, p)) t *= 1.10;
+    if (v.workspace) t += (double(g.M) + double(g.N)) * double(g.K) * (p.kind == ICL_KIND_CGEMM ? 16.0 : 8.0) / 5e12;
     return (float)(1.0 / t);
 }
 
@@ -135,38 +128,74 @@ const icl_gemm_variant* gemm_select(iclblasContext* h, const GemmProblem& p)
     return gemm_best(p);
 }
 
-// The three-way split kernels are candidates from a packed depth of 256 (k, or 2 k
-// of a complex product) on. Real products of up to 2 G multiply-adds stay on FP32
-// MFMA, so that iclblasSgemmNoAlloc, which has no workspace for the split, gives
-// iclblasSgemm's bits there (1024 x 1536 x 1024, 1.6 G: 46 us against about 40);
-// smaller complex ones than 0.5 G real multiply-adds take longer to pack than to
-// multiply. The workspace (12 bytes per padded element of op(A) and op(B)^T at most,
-// and 256 MiB of partial sums) is bounded.
-constexpr int kSplit3MinDepth = 256;
-constexpr double kSplit3MinMacs[2] = {2e9, 0.5e9}; // real multiply-adds of a real, a complex product
+// The three-way split kernels are candidates from a packed depth of 128 (k, or 2 k
+// of a complex product) and 0.1 G real multiply-adds on: the pack, the product and the
+// guarded kernel behind it take 20 us at the least. The workspace (12 bytes per padded
+// element of op(A) and op(B)^T at most, and 256 MiB of partial sums) is bounded.
+constexpr int kSplit3MinDepth = 128;
+constexpr double kSplit3MinMacs = 0.1e9;
 constexpr size_t kSplit3MaxBytes = size_t(8) << 30;
+static double real_macs(int kind, const icl_gemm_args& g)
+{
+    return (kind == ICL_KIND_CGEMM ? 4.0 : 1.0) * g.M * double(g.N) * g.K;
+}
 static bool split3_candidate(int kind, const icl_gemm_args& g)
 {
-    const int c = kind == ICL_KIND_CGEMM ? 2 : 1;
-    return c * g.K >= kSplit3MinDepth && double(c) * c * g.M * double(g.N) * g.K >= kSplit3MinMacs[c - 1];
+    return (kind == ICL_KIND_CGEMM ? 2 : 1) * g.K >= kSplit3MinDepth && real_macs(kind, g) >= kSplit3MinMacs;
+}
+
+// Whether a product that would run on the kernel `native` takes less time on
+// the packed kernel `split` of its math mode. The native time: the tiles of the busiest CU at
+// its full rate (alone on a CU a tile takes 1.25 times as long as its share of a full
+// one: it has one wave per SIMD), bounds-checked 1.9 (complex 1.6; split-BF16 1) and with a triangle
+// 1.25 times that, and 4 us. Against 120 random products the two estimates were off by
+// 10 and 13% and the choice lost 1% against the better of both (all on FP32 MFMA: 50%).
+// Real products of less than 2 G multiply-adds move only for a gain of a third: callers
+// without a workspace (iclblasSgemmNoAlloc, capped handles, captured streams) stay on
+// FP32 MFMA, and their results should differ from iclblasSgemm's only where it pays
+// (1024 x 1536 x 1024: 49 us against 40).
+static bool split_pays(const GemmProblem& p, const icl_gemm_variant& native, const icl_gemm_variant& split)
+{
+    const icl_gemm_args& g = *p.args;
+    const bool cplx = p.kind == ICL_KIND_CGEMM;
+    constexpr double kCUs = 256.0;
+    const double tiles = g.write_tri != ICL_TRI_NONE
+                             ? double(tri_tile_count(g.M, g.N, g.write_tri, native.bm, native.bn))
+                             : double((g.M + native.bm - 1) / native.bm) * double((g.N + native.bn - 1) / native.bn);
+    const double each = 2.0 * (cplx ? 4.0 : 1.0) * native.bm * native.bn * double(g.K) * kCUs / (native.tflops_hint * 1e12);
+    double t = tiles <= kCUs ? 1.25 * each : std::ceil(tiles / kCUs) * each;
+    if (g.kband != ICL_KBAND_NONE) t = std::max(1.25 * each, 0.5 * tiles / kCUs * each);
+    const bool fp32 = native.math == ICL_MATH_FP32;
+    if (fp32 && gemm_needs_edge(native, p)) t *= cplx ? 1.6 : 1.9;
+    if (g.write_tri != ICL_TRI_NONE) t *= 1.25;
+    const double margin = fp32 && !cplx && real_macs(p.kind, g) < 2e9 ? 1.33 : 1.0;
+    return t + 4e-6 > margin * split.estimate(&g);
 }
 
 // The accepted implementation with the highest score.
 static const icl_gemm_variant* gemm_best(const GemmProblem& p)
 {
-    const icl_gemm_variant* best = nullptr;
+    const icl_gemm_variant *best = nullptr, *split = nullptr;
     float best_score = -1.0f;
+    double split_time = 0.0;
+    const bool splits = p.optional_ws && split3_candidate(p.kind, *p.args);
     for (const icl_gemm_variant* v : gemm_registry()) {
         if (!gemm_accept(*v, p) || (p.no_ws && v->workspace)) continue;
-        if (v->math == ICL_MATH_FP32 && v->workspace &&
-            (!split3_candidate(p.kind, *p.args) || v->workspace(p.args) > kSplit3MaxBytes))
-            continue;
+        if (v->workspace && splits && v->workspace(p.args) <= kSplit3MaxBytes) {
+            const double t = v->estimate(p.args);
+            if (!split || t < split_time) {
+                split = v;
+                split_time = t;
+            }
+        }
+        if (v->workspace && v->math == ICL_MATH_FP32) continue;
         const float s = gemm_score(*v, p);
         if (s > best_score) {
             best = v;
             best_score = s;
         }
     }
+    if (best && split && !best->workspace && split_pays(p, *best, *split)) return split;
     if (!best) throw status_error(ICLBLAS_STATUS_NOT_SUPPORTED, "no GEMM implementation accepts the parameters");
     if (best->math != ICL_MATH_FP32 && best->workspace) { // of the packed ones, the one that estimates the shortest time
         double best_time = best->estimate(p.args);
@@ -257,7 +286,7 @@ static void run_gemm(iclblasContext* h, int kind, int math, int opa, int opb, ic
     if (math == ICL_MATH_BF16X3 && g.K < kSplitMinK) math = ICL_MATH_FP32;
     const hipStream_t s = stream ? stream : h->stream;
     GemmProblem p{kind, math, opa, opb, &g};
-    p.optional_ws = math == ICL_MATH_FP32 && optional_workspace(h, kind, g, s);
+    p.optional_ws = optional_workspace(h, kind, g, s);
     const icl_gemm_variant* v = gemm_select(h, p);
     if (level3_problem(g) && !v->level3)
         throw status_error(ICLBLAS_STATUS_INTERNAL_ERROR, "level-3 GEMM options on a kernel without them");
@@ -271,7 +300,6 @@ static void run_gemm(iclblasContext* h, int kind, int math, int opa, int opb, ic
         v = native;
     }
     if (v->workspace && h->budget.limit && !h->ext_ws) v = capped_variant(h, v, p, g);
-    const bool edge = gemm_needs_edge(*v, p);
     void* ws = nullptr;
     if (v->workspace) {
         if (h->ext_ws && v->workspace(&g) > h->ext_ws_bytes) g.whole_depth = 1;
@@ -281,9 +309,16 @@ static void run_gemm(iclblasContext* h, int kind, int math, int opa, int opb, ic
                 throw status_error(ICLBLAS_STATUS_INVALID_VALUE, "GEMM workspace exceeds the caller's scratch");
             ws = h->ext_ws;
         } else if (bytes) {
-            ws = h->scratch[iclblasContext::kSlotGemmWorkspace].get(bytes, h->stream);
+            icl::DeviceScratch& scratch = h->scratch[iclblasContext::kSlotGemmWorkspace];
+            if (p.optional_ws) ws = scratch.try_get(bytes, h->stream);
+            if (!ws) {
+                p.optional_ws = false; // the implementation that needs no more than it must
+                v = h->forced_impl.empty() && !h->budget.limit ? gemm_best(p) : v;
+                if (v->workspace) ws = scratch.get(v->workspace(&g), h->stream);
+            }
         }
     }
+    const bool edge = gemm_needs_edge(*v, p);
     // A variant with a prepass marks its main kernel itself (icl_timer_mark),
     // and may run half of the prepass on the handle's side stream: offered for
     // products of at least 1024 tiles of that variant, never to a call that must

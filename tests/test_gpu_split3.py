@@ -208,3 +208,42 @@ def test_sums_of_squares_lose_nothing(h, impl):
         h.set_memory_mode(ib.MEMORY_HOST)
     off = ((C.diag().double() - E) / E).mean().abs().item()
     assert off <= 2.0 ** -23 + 5 * U32 * (k / 32) ** 0.5 / n ** 0.5
+
+
+def _split_handle(cap):
+    import torch
+    h = ib.Handle(memory_mode=ib.MEMORY_DEVICE, math_mode=ib.MATH_SPLIT_BF16X3,
+                  stream=torch.cuda.current_stream().cuda_stream)
+    h.set_scratch_limit(cap)
+    return h
+
+
+@pytest.mark.parametrize("cplx,n,cap,impl", [
+    (False, 1024, 8 << 20, "sgemm_bf16x3d"),  # just the packed operands, no partial sums
+    (True, 2048, 80 << 20, "cgemm_bf16x3_"),  # 64 MiB packed once, 96 MiB with op(A) packed as rows of two
+    (True, 2048, 96 << 20, "cgemm_bf16x3d"),
+    (True, 2048, 60 << 20, None)])
+def test_split_bf16_under_a_cap(cplx, n, cap, impl):
+    """A capped handle's split-BF16 products: what the packed operands fit runs, what they do not is refused."""
+    rnd = np.random.default_rng(8)
+    A, B = (rnd.standard_normal((n, n)).astype(np.float32) for _ in range(2))
+    if cplx:
+        A, B = (X + 1j * rnd.standard_normal((n, n)).astype(np.float32) for X in (A, B))
+    tA, tB = _dev(A), _dev(B)
+    import torch
+    C = torch.zeros_like(tA)
+    with _split_handle(cap) as h:
+        f = ib.iclblasCgemm if cplx else ib.iclblasSgemm
+        st = f(h.value, 0, 0, n, n, n, 1.0, tA.data_ptr(), n, tB.data_ptr(), n, 0.0, C.data_ptr(), n)
+        h.synchronize()
+        if impl is None:
+            assert st == ib.STATUS_ALLOC_FAILED and not C.any()
+            return
+        ib.check(st)
+        assert h.last_implementation().startswith(impl)
+        assert h.scratch_usage()[0] <= cap
+    W = np.complex128 if cplx else np.float64
+    E = A.astype(W) @ B.astype(W)
+    ab = np.abs(A).astype(np.float64) @ np.abs(B).astype(np.float64)
+    c = 2 if cplx else 1
+    assert bound_ratio(np.abs(C.cpu().numpy().T.astype(W) - E), c * n, c * ab) <= 4.0
