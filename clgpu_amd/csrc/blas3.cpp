@@ -73,7 +73,7 @@ bool gemm_needs_edge(const icl_gemm_variant& v, const GemmProblem& p)
 // 5 TB/s). The bounds-checked instantiation is taken to run 10% slower: this ranks
 // implementations of one kind; whether a split-BF16 product needs a workspace, which a
 // handle's cap may refuse, hangs on these figures too. FP32 products on the three-way
-// split kernels are chosen by split_pays.
+// split kernels are chosen in gemm_best.
 // For K <= 512 a tile's fixed cost (pipeline fill, C read and write) is no
 // longer small against its K loop: it is counted as kTileOverheadK * (elements
 // of C per wave) extra steps of K, normalised so that the rate at K = 8192 is
@@ -144,43 +144,39 @@ static bool split3_candidate(int kind, const icl_gemm_args& g)
     return (kind == ICL_KIND_CGEMM ? 2 : 1) * g.K >= kSplit3MinDepth && real_macs(kind, g) >= kSplit3MinMacs;
 }
 
-// Whether a product that would run on the kernel `native` takes less time on
-// the packed kernel `split` of its math mode. The native time: the tiles of the busiest CU at
-// its full rate (alone on a CU a tile takes 1.25 times as long as its share of a full
-// one: it has one wave per SIMD), bounds-checked 1.9 (complex 1.6; split-BF16 1) and with a triangle
-// 1.25 times that, and 4 us. Against 120 random products the two estimates were off by
-// 10 and 13% and the choice lost 1% against the better of both (all on FP32 MFMA: 50%).
-// Real products of less than 2 G multiply-adds move only for a gain of a third: callers
-// without a workspace (iclblasSgemmNoAlloc, capped handles, captured streams) stay on
-// FP32 MFMA, and their results should differ from iclblasSgemm's only where it pays
-// (1024 x 1536 x 1024: 49 us against 40).
-static bool split_pays(const GemmProblem& p, const icl_gemm_variant& native, const icl_gemm_variant& split)
+// Seconds a product takes on a tiled kernel without a prepass: the tiles of the busiest
+// CU at its full rate (alone on a CU a tile takes 1.25 times as long as its share of a
+// full one: it has one wave per SIMD), FP32 bounds-checked 1.9 (complex 1.6) and with a
+// triangle 1.25 times that, and 4 us. Against 120 random products this was off by 13%.
+static double tiled_time(const GemmProblem& p, const icl_gemm_variant& v)
 {
     const icl_gemm_args& g = *p.args;
     const bool cplx = p.kind == ICL_KIND_CGEMM;
     constexpr double kCUs = 256.0;
     const double tiles = g.write_tri != ICL_TRI_NONE
-                             ? double(tri_tile_count(g.M, g.N, g.write_tri, native.bm, native.bn))
-                             : double((g.M + native.bm - 1) / native.bm) * double((g.N + native.bn - 1) / native.bn);
-    const double each = 2.0 * (cplx ? 4.0 : 1.0) * native.bm * native.bn * double(g.K) * kCUs / (native.tflops_hint * 1e12);
+                             ? double(tri_tile_count(g.M, g.N, g.write_tri, v.bm, v.bn))
+                             : double((g.M + v.bm - 1) / v.bm) * double((g.N + v.bn - 1) / v.bn);
+    const double each = 2.0 * (cplx ? 4.0 : 1.0) * v.bm * v.bn * double(g.K) * kCUs / (v.tflops_hint * 1e12);
     double t = tiles <= kCUs ? 1.25 * each : std::ceil(tiles / kCUs) * each;
     if (g.kband != ICL_KBAND_NONE) t = std::max(1.25 * each, 0.5 * tiles / kCUs * each);
-    const bool fp32 = native.math == ICL_MATH_FP32;
-    if (fp32 && gemm_needs_edge(native, p)) t *= cplx ? 1.6 : 1.9;
+    if (v.math == ICL_MATH_FP32 && gemm_needs_edge(v, p)) t *= cplx ? 1.6 : 1.9;
     if (g.write_tri != ICL_TRI_NONE) t *= 1.25;
-    const double margin = fp32 && !cplx && real_macs(p.kind, g) < 2e9 ? 1.33 : 1.0;
-    return t + 4e-6 > margin * split.estimate(&g);
+    return t + 4e-6;
 }
 
 // The accepted implementation with the highest score.
 static const icl_gemm_variant* gemm_best(const GemmProblem& p)
 {
-    const icl_gemm_variant *best = nullptr, *split = nullptr;
+    const icl_gemm_variant *best = nullptr, *split = nullptr, *wave = nullptr;
     float best_score = -1.0f;
     double split_time = 0.0;
     const bool splits = p.optional_ws && split3_candidate(p.kind, *p.args);
     for (const icl_gemm_variant* v : gemm_registry()) {
         if (!gemm_accept(*v, p) || (p.no_ws && v->workspace)) continue;
+        if (!v->workspace && v->estimate) {
+            wave = v;
+            continue;
+        }
         if (v->workspace && splits && v->workspace(p.args) <= kSplit3MaxBytes) {
             const double t = v->estimate(p.args);
             if (!split || t < split_time) {
@@ -195,7 +191,23 @@ static const icl_gemm_variant* gemm_best(const GemmProblem& p)
             best_score = s;
         }
     }
-    if (best && split && !best->workspace && split_pays(p, *best, *split)) return split;
+    if (best && !best->workspace && (wave || split)) {
+        // The estimates of the three families. Real FP32 products of less than 2 G
+        // multiply-adds move to the packed kernels only for a gain of a third: callers
+        // without a workspace (iclblasSgemmNoAlloc, capped handles, captured streams)
+        // cannot, and their results should differ from iclblasSgemm's only where it pays
+        // (1024 x 1536 x 1024: 49 us against 40). Chosen so, 120 random products lost 1%
+        // against the fastest kernel of each (all on FP32 MFMA tiles: 50%).
+        double t = tiled_time(p, *best);
+        if (wave && wave->estimate(p.args) < 0.9 * t) {
+            best = wave;
+            t = wave->estimate(p.args);
+        }
+        const double margin = best->math == ICL_MATH_FP32 && p.kind == ICL_KIND_SGEMM && real_macs(p.kind, *p.args) < 2e9 ? 1.33
+                              : p.args->write_tri != ICL_TRI_NONE ? 1.25 // tiled_time is high for short triangles
+                                                                  : 1.0;
+        if (split && t > margin * split_time) return split;
+    }
     if (!best) throw status_error(ICLBLAS_STATUS_NOT_SUPPORTED, "no GEMM implementation accepts the parameters");
     if (best->math != ICL_MATH_FP32 && best->workspace) { // of the packed ones, the one that estimates the shortest time
         double best_time = best->estimate(p.args);

@@ -750,7 +750,7 @@ double sp_estimate(const icl_gemm_args* g)
 {
     const SplitLayout l = sp_layout<T, PLANES, CPLX>(g);
     const double read = (CPLX ? 8.0 : 4.0) * (double(g->M) + g->N) * g->K;
-    double us = (read + l.a_bytes + l.b_bytes) / 4.8e6 + l.plan.us + l.band.us + (PLANES == 3 ? 8.0 : 3.0);
+    double us = (read + l.a_bytes + l.b_bytes) / 4.8e6 + l.plan.us + l.band.us + (PLANES == 3 ? 10.0 : 3.0);
     return us * 1e-6;
 }
 
