@@ -186,17 +186,21 @@ __global__ void __launch_bounds__(256) ctrsm_invert_kernel(icl_ctrsm_blocked_arg
                 const int blk = e / (h * h), rc = e % (h * h), r = rc / h, c = rc % h;
                 const int o = blk * 2 * h;
                 float2 acc = make_float2(0.0f, 0.0f);
+                // Every k with a select, not k from c or up to r: the loop's reads then run
+                // ahead of the sums (a variable bound made each step wait for LDS).
                 if (step == 0) { // T(r, c) = sum_k C(r, k) inv(A)(k, c), k >= c
-                    for (int k = c; k < h; ++k) {
+#pragma unroll 8
+                    for (int k = 0; k < h; ++k) {
                         const float2 t = c_mul(Ls[o + h + r][o + k], Is[o + k][o + c]);
-                        acc.x += t.x;
-                        acc.y += t.y;
+                        acc.x += k >= c ? t.x : 0.0f;
+                        acc.y += k >= c ? t.y : 0.0f;
                     }
                 } else { // -sum_k inv(D)(r, k) T(k, c), k <= r
-                    for (int k = 0; k <= r; ++k) {
+#pragma unroll 8
+                    for (int k = 0; k < h; ++k) {
                         const float2 t = c_mul(Is[o + h + r][o + h + k], Ts[blk * h + k][c]);
-                        acc.x -= t.x;
-                        acc.y -= t.y;
+                        acc.x -= k <= r ? t.x : 0.0f;
+                        acc.y -= k <= r ? t.y : 0.0f;
                     }
                 }
                 out[q] = acc;
@@ -327,13 +331,18 @@ __global__ void __launch_bounds__(kApThreads) ctrsm_apply_kernel(icl_ctrsm_apply
 //  level 2, workgroup (p, q): W_rc = -sum_{k = 2..r} W_rk T_kc, i.e. -inv(D) T.
 // The longest chain is two 64 x 64 x 64 complex products per launch, where
 // building the column blocks one after the other (M_ij = -iD_i sum_{k=j}^{i-1}
-// L_ik M_kj) chains nine. Each product runs on v_mfma_f32_32x32x2_f32 with the
-// operands staged in LDS as planar re / im tiles, A as [k][row] and B as
-// [k][col], each of the four waves owning a 32 x 32 quadrant.
+// L_ik M_kj) chains nine. A workgroup forms a 32 x 32 quadrant of a block, each of its
+// four waves a quarter of every product's depth on v_mfma_f32_32x32x2_f32, from
+// operands staged in LDS as planar re / im tiles, A as [k][row] and B as [k][col]; the
+// four partial sums are added in order through LDS. (One workgroup per block kept its
+// matrix cores busy 3.6 us per product on 2 or 4 CUs per panel: 33 + 18 + 18 us for
+// order 1153.)
 constexpr int kPanRows = 256;
-constexpr int kPnLd = kNB + 1;
-constexpr size_t kPanInvLds = sizeof(float) * 4 * kNB * kPnLd;
-constexpr int kPer = kNB * kNB / 256; // elements of a 64 x 64 block per thread; e = tid + 256 q: (x = e % 64, y = e / 64)
+constexpr int kPnQ = 32;         // quadrant
+constexpr int kPnLd = kPnQ + 1;
+constexpr int kPnWaves = 4;
+constexpr size_t kPanInvLds = sizeof(float) * (4 * kNB + 2 * kPnWaves * kPnQ) * kPnLd;
+constexpr int kPer = kPnQ * kNB / 256; // elements of half a 64 x 64 block per thread
 
 // A 64 x 64 operand block: element (x, y) of the block.
 struct PanBlk {
@@ -352,17 +361,20 @@ struct PanCtx {
                      : (long)r * a.w_rs + (long)c * a.w_cs;
     }
     __device__ float2* t_blk(int r, int c) const { return T + ((long)pnl * 4 + (r - 2) * 2 + c) * kNB * kNB; }
-    // All loads first, unconditionally (an entry outside the system or the panel
-    // reads element 0 of its array instead and is replaced by 0 afterwards).
-    __device__ void load(const PanBlk& b, int tid, float2 (&v)[kPer]) const
+    // Elements e = tid + 256 q of the block's part of NX rows from x0 on and the columns
+    // from y0 on, (x, y) = (x0 + e % NX, y0 + e / NX). All loads first, unconditionally
+    // (an entry outside the system or the panel reads element 0 of its array instead and
+    // is replaced by 0 afterwards).
+    template <int NX, int N>
+    __device__ void load(const PanBlk& b, int tid, int x0, int y0, float2 (&v)[N]) const
     {
         const float2* L = reinterpret_cast<const float2*>(a.L);
         const float2* invD = reinterpret_cast<const float2*>(a.invD);
         const float sg = a.conj ? -1.0f : 1.0f;
-        bool ok[kPer];
+        bool ok[N];
 #pragma unroll
-        for (int q = 0; q < kPer; ++q) {
-            const int e = tid + 256 * q, x = e % kNB, y = e / kNB;
+        for (int q = 0; q < N; ++q) {
+            const int e = tid + 256 * q, x = x0 + e % NX, y = y0 + e / NX;
             const int r = kNB * b.bi + x, c = kNB * b.bj + y;
             switch (b.kind) {
             case PanBlk::L:
@@ -385,11 +397,12 @@ struct PanCtx {
             }
         }
 #pragma unroll
-        for (int q = 0; q < kPer; ++q)
+        for (int q = 0; q < N; ++q)
             if (!ok[q]) v[q] = make_float2(0.0f, 0.0f);
     }
 };
 
+// Workgroup (panel, block, quadrant).
 __global__ void __launch_bounds__(256) ctrsm_invert_panels_kernel(icl_ctrsm_panel_inv_args a, int level)
 {
     extern __shared__ float sm[];
@@ -397,58 +410,87 @@ __global__ void __launch_bounds__(256) ctrsm_invert_panels_kernel(icl_ctrsm_pane
     float(*Ai)[kPnLd] = Ar + kNB;
     float(*Br)[kPnLd] = Ai + kNB; // B[k][col]
     float(*Bi)[kPnLd] = Br + kNB;
+    float(*part)[kPnLd] = Bi + kNB; // [(2 wave + re / im) * 32 + col][row]
     const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
-    const int wr = 32 * (wave & 1), wc = 32 * (wave >> 1);
+    const int quad = blockIdx.z, wr = kPnQ * (quad & 1), wc = kPnQ * (quad >> 1);
     const int pnl = blockIdx.x, ps = pnl * kPanRows;
     const int plen = min(kPanRows, a.nsys - ps), nb = (plen + kNB - 1) / kNB;
     const PanCtx cx{a, pnl, ps, plen, reinterpret_cast<float2*>(a.W) + (long)pnl * kPanRows * kPanRows,
                     reinterpret_cast<float2*>(a.T)};
 
-    // Stage X as the A tile and Y as the B tile (after a barrier, so no wave still
-    // reads the previous tiles), then acc (+)= X Y; lanes along rows of the result.
-    auto product = [&](const PanBlk& X, const PanBlk& Y, f32x16& accr, f32x16& acci) {
-        float2 va[kPer], vb[kPer];
-        cx.load(X, tid, va);
-        cx.load(Y, tid, vb);
-        __syncthreads();
+    auto stage_a = [&](const float2 (&v)[kPer]) { // rows of the quadrant, all k
 #pragma unroll
         for (int q = 0; q < kPer; ++q) {
-            const int e = tid + 256 * q, x = e % kNB, y = e / kNB; // X: (row x, k y); Y: (k x, col y)
-            Ar[y][x] = va[q].x;
-            Ai[y][x] = va[q].y;
-            Br[x][y] = vb[q].x;
-            Bi[x][y] = vb[q].y;
+            const int e = tid + 256 * q;
+            Ar[e / kPnQ][e % kPnQ] = v[q].x;
+            Ai[e / kPnQ][e % kPnQ] = v[q].y;
         }
-        __syncthreads();
-#pragma unroll 8
-        for (int kk = 0; kk < kNB; kk += 2) {
-            const int kr = kk + (lane >> 5);
-            const float ar = Ar[kr][wr + (lane & 31)], ai = Ai[kr][wr + (lane & 31)];
-            const float br = Br[kr][wc + (lane & 31)], bi = Bi[kr][wc + (lane & 31)];
+    };
+    // accr, acci += this wave's quarter of the depth of A B; lanes along A's rows.
+    auto multiply = [&](f32x16& accr, f32x16& acci) {
+#pragma unroll
+        for (int kk = 0; kk < kNB / kPnWaves; kk += 2) {
+            const int kr = kNB / kPnWaves * wave + kk + (lane >> 5);
+            const float ar = Ar[kr][lane & 31], ai = Ai[kr][lane & 31];
+            const float br = Br[kr][lane & 31], bi = Bi[kr][lane & 31];
             accr = icl::mfma_32x32x2_f32(br, ar, accr);
             acci = icl::mfma_32x32x2_f32(bi, ar, acci);
             accr = icl::mfma_32x32x2_f32(bi, -ai, accr);
             acci = icl::mfma_32x32x2_f32(br, ai, acci);
         }
     };
-    // Element (row, col) of this lane's accumulator entry r.
-    auto row_of = [&](int) { return wr + (lane & 31); };
-    auto col_of = [&](int r) { return wc + icl::mfma32_row(lane, r); };
-    auto store_w = [&](int bi, int bj, const f32x16& accr, const f32x16& acci, float s) {
-#pragma unroll
-        for (int r = 0; r < 16; ++r) {
-            const int row = kNB * bi + row_of(r), col = kNB * bj + col_of(r);
-            if (row < plen && col < plen) cx.W[cx.w_at(row, col)] = make_float2(s * accr[r], s * acci[r]);
-        }
-    };
-    auto copy_w = [&](const PanBlk& src, int bi, int bj) { // W_(bi, bj) = src (zero when src is null)
-        float2 v[kPer];
-        if (src.kind == PanBlk::INVD) cx.load(src, tid, v);
-        else
-            for (int q = 0; q < kPer; ++q) v[q] = make_float2(0.0f, 0.0f);
+    // Stage X's rows from r0 on as the A tile and Y's columns of the quadrant as the B
+    // tile (after a barrier, so no wave still reads the previous tiles), then acc (+)= X Y.
+    auto product = [&](const PanBlk& X, int r0, const PanBlk& Y, f32x16& accr, f32x16& acci) {
+        float2 va[kPer], vb[kPer];
+        cx.load<kPnQ>(X, tid, r0, 0, va);
+        cx.load<kNB>(Y, tid, 0, wc, vb);
+        __syncthreads();
+        stage_a(va);
 #pragma unroll
         for (int q = 0; q < kPer; ++q) {
-            const int e = tid + 256 * q, r = kNB * bi + e % kNB, c = kNB * bj + e / kNB;
+            const int e = tid + 256 * q;
+            Br[e % kNB][e / kNB] = vb[q].x;
+            Bi[e % kNB][e / kNB] = vb[q].y;
+        }
+        __syncthreads();
+        multiply(accr, acci);
+    };
+    // The waves' sums, added: out[i] = element (row tid % 32, column tid / 32 + 8 i) of the quadrant.
+    auto reduce = [&](const f32x16& accr, const f32x16& acci, float2 (&out)[4]) {
+        __syncthreads();
+#pragma unroll
+        for (int r = 0; r < 16; ++r) {
+            part[(2 * wave) * kPnQ + icl::mfma32_row(lane, r)][lane & 31] = accr[r];
+            part[(2 * wave + 1) * kPnQ + icl::mfma32_row(lane, r)][lane & 31] = acci[r];
+        }
+        __syncthreads();
+#pragma unroll
+        for (int i = 0; i < 4; ++i) {
+            const int row = tid & 31, col = (tid >> 5) + 8 * i;
+            out[i] = make_float2(0.0f, 0.0f);
+#pragma unroll
+            for (int w = 0; w < kPnWaves; ++w) {
+                out[i].x += part[(2 * w) * kPnQ + col][row];
+                out[i].y += part[(2 * w + 1) * kPnQ + col][row];
+            }
+        }
+    };
+    auto store_w = [&](int bi, int bj, const float2 (&v)[4], float s) {
+#pragma unroll
+        for (int i = 0; i < 4; ++i) {
+            const int row = kNB * bi + wr + (tid & 31), col = kNB * bj + wc + (tid >> 5) + 8 * i;
+            if (row < plen && col < plen) cx.W[cx.w_at(row, col)] = make_float2(s * v[i].x, s * v[i].y);
+        }
+    };
+    auto copy_w = [&](const PanBlk& src, int bi, int bj) { // this quadrant's columns of W_(bi, bj) = src (or zero)
+        float2 v[4];
+        if (src.kind == PanBlk::INVD) cx.load<kNB>(src, tid, 0, 16 * quad, v);
+        else
+            for (int q = 0; q < 4; ++q) v[q] = make_float2(0.0f, 0.0f);
+#pragma unroll
+        for (int q = 0; q < 4; ++q) {
+            const int e = tid + 256 * q, r = kNB * bi + e % kNB, c = kNB * bj + 16 * quad + e / kNB;
             if (r < plen && c < plen) cx.W[cx.w_at(r, c)] = v[q];
         }
     };
@@ -464,51 +506,49 @@ __global__ void __launch_bounds__(256) ctrsm_invert_panels_kernel(icl_ctrsm_pane
                 for (int j = 2; j < 4; ++j) copy_w(zero, i, j);
         if (dd >= nb) return;
         copy_w({PanBlk::INVD, dd, dd}, dd, dd);
+        // The quadrant's columns of S = L_da iD_a, 64 rows, in two halves.
+        float2 s0[4], s1[4], vd[kPer];
         f32x16 sr = f32x16{}, si = f32x16{};
-        product({PanBlk::L, dd, da}, {PanBlk::INVD, da, da}, sr, si); // S = L_da iD_a
-        // W_da = -iD_d S: S becomes the B tile, iD_d the A tile.
-        float2 vd[kPer];
-        cx.load({PanBlk::INVD, dd, dd}, tid, vd);
+        product({PanBlk::L, dd, da}, 0, {PanBlk::INVD, da, da}, sr, si);
+        reduce(sr, si, s0);
+        sr = f32x16{}, si = f32x16{};
+        product({PanBlk::L, dd, da}, kPnQ, {PanBlk::INVD, da, da}, sr, si);
+        reduce(sr, si, s1);
+        // W_da = -iD_d S: S becomes the B tile, iD_d's rows the A tile.
+        cx.load<kPnQ>({PanBlk::INVD, dd, dd}, tid, wr, 0, vd);
         __syncthreads();
 #pragma unroll
-        for (int r = 0; r < 16; ++r) {
-            Br[row_of(r)][col_of(r)] = sr[r];
-            Bi[row_of(r)][col_of(r)] = si[r];
+        for (int i = 0; i < 4; ++i) {
+            const int row = tid & 31, col = (tid >> 5) + 8 * i;
+            Br[row][col] = s0[i].x;
+            Bi[row][col] = s0[i].y;
+            Br[kPnQ + row][col] = s1[i].x;
+            Bi[kPnQ + row][col] = s1[i].y;
         }
-#pragma unroll
-        for (int q = 0; q < kPer; ++q) {
-            const int e = tid + 256 * q, x = e % kNB, y = e / kNB;
-            Ar[y][x] = vd[q].x;
-            Ai[y][x] = vd[q].y;
-        }
+        stage_a(vd);
         __syncthreads();
-        f32x16 mr = f32x16{}, mi = f32x16{};
-#pragma unroll 8
-        for (int kk = 0; kk < kNB; kk += 2) {
-            const int kr = kk + (lane >> 5);
-            const float ar = Ar[kr][wr + (lane & 31)], ai = Ai[kr][wr + (lane & 31)];
-            const float br = Br[kr][wc + (lane & 31)], bi = Bi[kr][wc + (lane & 31)];
-            mr = icl::mfma_32x32x2_f32(br, ar, mr);
-            mi = icl::mfma_32x32x2_f32(bi, ar, mi);
-            mr = icl::mfma_32x32x2_f32(bi, -ai, mr);
-            mi = icl::mfma_32x32x2_f32(br, ai, mi);
-        }
-        store_w(dd, da, mr, mi, -1.0f);
+        sr = f32x16{}, si = f32x16{};
+        multiply(sr, si);
+        reduce(sr, si, s0);
+        store_w(dd, da, s0, -1.0f);
         return;
     }
     const int q = blockIdx.y, r = 2 + (q >> 1), c = q & 1;
     if (r >= nb) return;
     f32x16 accr = f32x16{}, acci = f32x16{};
+    float2 out[4];
     if (level == 1) { // T_rc = sum_{k = c..1} L_rk W_kc
-        for (int k = c; k < 2; ++k) product({PanBlk::L, r, k}, {PanBlk::WBLK, k, c}, accr, acci);
+        for (int k = c; k < 2; ++k) product({PanBlk::L, r, k}, wr, {PanBlk::WBLK, k, c}, accr, acci);
+        reduce(accr, acci, out);
         float2* t = cx.t_blk(r, c);
 #pragma unroll
-        for (int e = 0; e < 16; ++e) t[(long)col_of(e) * kNB + row_of(e)] = make_float2(accr[e], acci[e]);
+        for (int i = 0; i < 4; ++i) t[(long)(wc + (tid >> 5) + 8 * i) * kNB + wr + (tid & 31)] = out[i];
         return;
     }
     // level 2: W_rc = -sum_{k = 2..r} W_rk T_kc
-    for (int k = 2; k <= r; ++k) product({PanBlk::WBLK, r, k}, {PanBlk::TBLK, k, c}, accr, acci);
-    store_w(r, c, accr, acci, -1.0f);
+    for (int k = 2; k <= r; ++k) product({PanBlk::WBLK, r, k}, wr, {PanBlk::TBLK, k, c}, accr, acci);
+    reduce(accr, acci, out);
+    store_w(r, c, out, -1.0f);
 }
 
 } // namespace
@@ -521,7 +561,7 @@ extern "C" hipError_t icl_ctrsm_invert_panels(const icl_ctrsm_panel_inv_args* a,
     if (attr != hipSuccess) return attr;
     const unsigned panels = (unsigned)((a->nsys + kPanRows - 1) / kPanRows);
     for (int level = 0; level < 3; ++level) {
-        hipLaunchKernelGGL(ctrsm_invert_panels_kernel, dim3(panels, level == 0 ? 2 : 4), dim3(256), kPanInvLds, stream,
+        hipLaunchKernelGGL(ctrsm_invert_panels_kernel, dim3(panels, level == 0 ? 2 : 4, 4), dim3(256), kPanInvLds, stream,
                            *a, level);
         const hipError_t e = hipGetLastError();
         if (e != hipSuccess) return e;
