@@ -236,23 +236,20 @@ __device__ __forceinline__ void sp_products(const bf16x8 (&b)[FN], bf16x8 a, f32
         t[j] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(b[j], a, FIRST ? f32x4{} : t[j], 0, 0, 0);
 }
 
-// c += a b in place: v_mfma_f32_16x16x32_bf16 with the sum's registers tied. Written
-// out because the compiler gives each of the builtin's results registers of its own
-// and then has too few left for operands read ahead (256 per wave: 128 hold sums).
-// It does not see the instruction's latency: a sum is used again only by a product
-// at least FM * FN instructions later, or after sp_drain.
+// c += a b. The builtin, not an asm statement: the compiler knows its latency and the
+// waits that it needs before its operands are written and its sum is read.
 // Lane l supplies a = A[l % 16][8 (l / 16) .. + 7] and b = B[8 (l / 16) .. + 7][l % 16];
 // register r of c is D[4 (l / 16) + r][l % 16].
 __device__ __forceinline__ void sp_mfma1(bf16x8 a, bf16x8 b, f32x4& c)
 {
-    asm("v_mfma_f32_16x16x32_bf16 %0, %1, %2, %0" : "+v"(c) : "v"(a), "v"(b));
+    c = __builtin_amdgcn_mfma_f32_16x16x32_bf16(a, b, c, 0, 0, 0);
 }
 
-// Lets the last products finish before their sums are read, and the last copies.
+// Waits for the last copies: LDS may be another workgroup's after this one's end.
 __device__ __forceinline__ void sp_drain()
 {
     __builtin_amdgcn_sched_barrier(0);
-    asm volatile("s_waitcnt vmcnt(0)\n\ts_nop 15\n\ts_nop 15" ::: "memory");
+    asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
     __builtin_amdgcn_sched_barrier(0);
 }
 
