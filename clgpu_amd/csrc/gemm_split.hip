@@ -35,6 +35,7 @@
 #include "gemm_variants.hpp"
 
 #include <algorithm>
+#include <climits>
 #include <type_traits>
 
 namespace icl {
@@ -404,7 +405,7 @@ __global__ void __launch_bounds__(WVM* WVN * 64, T == 256 ? 2 : 4) split_gemm_ke
 
     // This wave's copies of a block: the k groups wave / RB + (NW / RB) i of 64 rows.
     const size_t a_row = (size_t)p.Mpad * 16, b_row = (size_t)p.Npad * 16; // bytes of one k group of all rows
-    const size_t a_slab = PLANES * kGroups * a_row, b_slab = PLANES * kGroups * b_row;
+    const size_t a_plane = kGroups * a_row, b_plane = kGroups * b_row, a_slab = PLANES * a_plane, b_slab = PLANES * b_plane;
     const char* a_src = reinterpret_cast<const char*>(p.Ap) + (size_t)ks0 * a_slab + (wave / Cfg::RB) * a_row +
                         (size_t)(m0 + 64 * (wave % Cfg::RB)) * 16;
     const char* b_src = reinterpret_cast<const char*>(p.Bp) + (size_t)ks0 * b_slab + (wave / Cfg::RB) * b_row +
@@ -414,15 +415,18 @@ __global__ void __launch_bounds__(WVM* WVN * 64, T == 256 ? 2 : 4) split_gemm_ke
     // Part `i` of the copy of a slab's block c to the ring slot at `slot` (bytes), src
     // being the slab's first byte of op(A) / op(B). A buffer load: its address stays
     // scalar, and a global load would count as a FLAT access, after which the compiler
-    // waits for all LDS reads at once.
+    // waits for all LDS reads at once. The plane is part of the 64-bit base and the
+    // descriptor unbounded: a slab of all rows is longer than 32-bit offsets and extents
+    // reach from 2^24 (three planes) or 2^25 rows on. What is left of the offset, 32 bytes
+    // per row, is checked by the launcher.
     constexpr int PER_SLAB = 2 * PLANES, KSTEP = Cfg::NW / Cfg::RB;
     auto copy = [&](const char* a, const char* b, int c, int slot, int i) {
         const bool of_a = PLANES == 3 ? c >= 3 : (c == 0 || c == 2);
         const int plane = PLANES == 3 ? (c < 3 ? 2 - c : c - 3) : (c == 0 || c == 3 ? 1 : 0);
-        const auto rsrc = __builtin_amdgcn_make_buffer_rsrc(const_cast<char*>(of_a ? a : b), 0,
-                                                            (unsigned)(of_a ? a_slab : b_slab), 0x20000);
+        const char* src = of_a ? a + plane * a_plane : b + plane * b_plane;
+        const auto rsrc = __builtin_amdgcn_make_buffer_rsrc(const_cast<char*>(src), 0, 0xffffffffu, 0x20000);
         __builtin_amdgcn_raw_ptr_buffer_load_lds(rsrc, (sp_lds_void*)(lds_sp + slot + (wave + Cfg::NW * i) * 1024), 16,
-                                                 loff, (kGroups * plane + KSTEP * i) * (int)(of_a ? a_row : b_row), 0, 0);
+                                                 loff, KSTEP * i * (unsigned)(of_a ? a_row : b_row), 0, 0);
     };
 
     f32x4 acc[Cfg::FM][Cfg::FN];
@@ -792,6 +796,7 @@ hipError_t sp_launch(const icl_gemm_args* g, int opa, int opb, int edge, void* w
     (void)edge;
     if (!ws || (PLANES == 3 && !g->guard)) return hipErrorInvalidValue;
     const SplitLayout l = sp_layout<T, PLANES, CPLX>(g);
+    if (32.0 * std::max(l.Mpad, l.Npad) > UINT_MAX) return hipErrorInvalidValue;
     SplitArgs p{};
     p.Mpad = l.Mpad;
     p.Npad = l.Npad;
