@@ -85,7 +85,8 @@ split_pack_kernel(SplitSrc a, SplitSrc b, int ablocks, int slabs, unsigned long 
     const bool is_a = (int)blockIdx.x < ablocks;
     const SplitSrc o = is_a ? a : b;
     const int r0 = (is_a ? (int)blockIdx.x : (int)blockIdx.x - ablocks) * 64; // packed row
-    const int k0 = blockIdx.y * 64;                                           // packed k
+    const int by = (int)(blockIdx.y + gridDim.y * blockIdx.z), k0 = by * 64;  // packed k
+    if (2 * by >= slabs) return; // the last layer of a deep grid
     const int t = threadIdx.x;
     bool bad = false;
     if constexpr (!CPLX) {
@@ -134,8 +135,8 @@ split_pack_kernel(SplitSrc a, SplitSrc b, int ablocks, int slabs, unsigned long 
     }
     if (PLANES == 3 && bad) *guard = epoch;
     __syncthreads();
-    // wave w writes k = 16 w .. 16 w + 15 of slab pair y, lane = row: 1 KB per store
-    const int w = t >> 6, r = t & 63, ks = 2 * (int)blockIdx.y + (w >> 1);
+    // wave w writes k = 16 w .. 16 w + 15 of slab pair by, lane = row: 1 KB per store
+    const int w = t >> 6, r = t & 63, ks = 2 * by + (w >> 1);
     if (ks >= slabs) return;
     bf16x8 out[PLANES][2];
 #pragma unroll
@@ -755,11 +756,14 @@ double sp_estimate(const icl_gemm_args* g)
     return us * 1e-6;
 }
 
-// Packs arows packed rows of `a` and brows of `b` (multiples of 64).
+// Packs arows packed rows of `a` and brows of `b` (multiples of 64). A grid's second
+// dimension ends at 65536 blocks, a depth of 2^22: deeper ones (FP32 products of few rows
+// reach 2^22.4) go on in the third.
 template <int PLANES, bool CPLX>
 hipError_t sp_pack(const SplitSrc& a, int arows, const SplitSrc& b, int brows, const SplitArgs& p, hipStream_t s)
 {
-    const dim3 grid((unsigned)((arows + brows) / 64), (unsigned)((p.slabs + 1) / 2));
+    const unsigned deep = (unsigned)((p.slabs + 1) / 2), layer = std::min(deep, 32768u);
+    const dim3 grid((unsigned)((arows + brows) / 64), layer, (deep + layer - 1) / layer);
     hipLaunchKernelGGL((split_pack_kernel<PLANES, CPLX>), grid, dim3(256), 0, s, a, b, arows / 64, p.slabs,
                        const_cast<unsigned long long*>(p.guard), p.epoch);
     return hipGetLastError();

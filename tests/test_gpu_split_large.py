@@ -1,5 +1,5 @@
 """The packed split kernels beyond 32-bit sizes: operands of more rows than a 32-bit extent
-of one slab reaches."""
+of one slab reaches, and depths of more slabs than a grid's second dimension holds."""
 import pytest
 
 from blas_helpers import U32
@@ -9,7 +9,7 @@ pytestmark = pytest.mark.gpu
 
 
 def _call(impl, ta, tb, m, n, k, A, lda, B, ldb, C, ldc):
-    """One SGEMM with `impl` (None: as selected) on a handle of its own."""
+    """One SGEMM with `impl` on a handle of its own."""
     import torch
     mode = ib.MATH_SPLIT_BF16X3 if "bf16x3" in impl else ib.MATH_FP32
     with ib.Handle(memory_mode=ib.MEMORY_DEVICE, math_mode=mode, stream=torch.cuda.current_stream().cuda_stream) as h:
@@ -42,3 +42,26 @@ def test_rows_past_the_32_bit_extent_of_a_slab(impl):
     assert bool(torch.isfinite(C).all())
     del A, B, C, X
     torch.cuda.empty_cache()
+
+
+@pytest.mark.parametrize("impl", ["sgemm_f32_split3_128x128", "sgemm_bf16x3d_mfma_128x128"])
+@pytest.mark.parametrize("ta,tb", [(0, 1), (1, 0)])
+def test_depth_past_the_grid_limit(impl, ta, tb):
+    """k = 2^22 + 100: 65538 pairs of slabs."""
+    import torch
+    m, n, k = 60, 70, (1 << 22) + 100
+    gen = torch.Generator("cuda").manual_seed(7)
+    A, B = (torch.empty((r, c), device="cuda").uniform_(-1, 1, generator=gen)
+            for r, c in (((k, m) if ta == 0 else (m, k)), ((n, k) if tb == 0 else (k, n))))
+    C = torch.full((n, m), float("nan"), device="cuda")
+    torch.cuda.synchronize()
+    _call(impl, ta, tb, m, n, k, A, A.shape[1], B, B.shape[1], C, m)
+    X, Y = (A.T if ta == 0 else A).double(), (B.T if tb == 0 else B).double()
+    err, mag = (C.T.double() - X @ Y).abs(), X.abs() @ Y.abs()
+    assert bool((err <= 4 * k * U32 * mag).all())
+    # the bound above grows with k: the last slabs, alone in a block of rows of zeros
+    A[(slice(0, 1 << 22), 0) if ta == 0 else (0, slice(0, 1 << 22))] = 0
+    _call(impl, ta, tb, m, n, k, A, A.shape[1], B, B.shape[1], C, m)
+    X = (A.T if ta == 0 else A).double()
+    err, mag = (C.T.double() - X @ Y).abs()[0], (X.abs() @ Y.abs())[0]
+    assert bool((err <= 4 * 256 * U32 * mag).all())
