@@ -287,12 +287,27 @@ __device__ __forceinline__ float sp_neighbour(float x)
         float, __builtin_amdgcn_mov_dpp(__builtin_bit_cast(int, x), 0xB1 /* quad_perm 1,0,3,2 */, 0xf, 0xf, true));
 }
 
+// Columns nl + c of a lane's row that are stored (or kept by a mask): those with
+// first <= nl + c < end, one subtraction and one comparison per element.
+struct SpColumns {
+    int from;
+    unsigned count;
+    __device__ __forceinline__ SpColumns(int nl, int first, int end)
+        : from(nl - first), count((unsigned)max(end - first, 0))
+    {
+    }
+    __device__ __forceinline__ bool has(int c) const { return (unsigned)(from + c) < count; }
+};
+
 // Stores G rows of FN 16 x 16 blocks, block row i at row0 + 16 i: register r of block j
 // holds column ncol0 + 16 j + 4 (lane / 16) + r, the lane row `row0` (complex: the part
 // lane & 1 of complex row row0 / 2). CHECK: bounds, triangle and mask are tested per
-// element. C is read for the whole group before anything is stored: row by row of blocks
-// each waited for memory again (2048 x 2048 x 256 with beta = 1: 35 us of 128 x 128
-// tiles, 12 of them products).
+// element, as a range of columns per row. C is read for the whole group before anything
+// is stored: row by row of blocks each waited for memory again (2048 x 2048 x 256 with
+// beta = 1: 35 us of 128 x 128 tiles, 12 of them products). The checked stores take 0.9
+// us of a call (100 x 90 x 256, two planes, 11.8 us; 128 x 128 x 256 10.9); each waiting
+// for the one before, their tests kept from the reads in spilled scalar registers, they
+// took 4.4.
 template <bool CPLX, bool CHECK, int G, int FN>
 __device__ __forceinline__ void sp_store(const GemmArgs& g, const f32x4 (&acc)[G][FN], int row0, int ncol0, int lane)
 {
@@ -301,26 +316,46 @@ __device__ __forceinline__ void sp_store(const GemmArgs& g, const f32x4 (&acc)[G
     float* const c0 = g.C + (CPLX ? 2L : 1L) * (long)nl * g.ldc + row0;
     const bool odd = CPLX && (lane & 1);
     const bool beta_zero = g.beta_re == 0.0f && (!CPLX || g.beta_im == 0.0f);
-    const TriMask tri(g.mask);
     auto m_of = [&](int i) { return (row0 + 16 * i) >> (CPLX ? 1 : 0); };
-    auto on = [&](int m, int n) { return !CHECK || (m < g.M && n < g.N && tri_writes(g.write_tri, m, n)); };
+    auto stored = [&](int i) {
+        const int m = m_of(i), tri = g.write_tri & 3;
+        return SpColumns(nl, tri == ICL_TRI_UPPER ? m : 0,
+                         !CHECK ? INT_MAX : m >= g.M ? 0 : tri == ICL_TRI_LOWER ? min(m + 1, g.N) : g.N);
+    };
+    auto kept = [&](int i) {
+        const int m = m_of(i), strict = g.mask == kMaskLowerStrict || g.mask == kMaskUpperStrict;
+        const bool lower = g.mask == kMaskLower || g.mask == kMaskLowerStrict;
+        return SpColumns(nl, g.mask == kMaskNone || lower ? 0 : m + strict, lower ? m + 1 - strict : INT_MAX);
+    };
     float old[G][FN][4];
     if (!beta_zero) {
+#pragma unroll
+        for (int i = 0; i < G; ++i) {
+            const SpColumns on = stored(i);
+#pragma unroll
+            for (int j = 0; j < FN; ++j)
+#pragma unroll
+                for (int r = 0; r < 4; ++r)
+                    old[i][j][r] = !CHECK || on.has(16 * j + r) ? c0[16 * i + (16 * j + r) * cstep] : 0.0f;
+        }
+        // Waited for here: left to their uses, the compiler waits at each of them, beta = 0
+        // or not, for everything outstanding, which by then is the store before it.
 #pragma unroll
         for (int i = 0; i < G; ++i)
 #pragma unroll
             for (int j = 0; j < FN; ++j)
 #pragma unroll
-                for (int r = 0; r < 4; ++r)
-                    old[i][j][r] = on(m_of(i), nl + 16 * j + r) ? c0[16 * i + (16 * j + r) * cstep] : 0.0f;
+                for (int r = 0; r < 4; ++r) asm volatile("" : "+v"(old[i][j][r]));
     }
 #pragma unroll
-    for (int i = 0; i < G; ++i)
+    for (int i = 0; i < G; ++i) {
+        SpColumns on = stored(i);
+        const SpColumns keep = kept(i);
+        if (CHECK) asm volatile("" : "+v"(on.from)); // tested again, not kept
 #pragma unroll
         for (int j = 0; j < FN; ++j)
 #pragma unroll
             for (int r = 0; r < 4; ++r) {
-                const int m = m_of(i), n = nl + 16 * j + r;
                 float v;
                 if constexpr (CPLX) {
                     // even lanes: alpha_re re - alpha_im im; odd lanes: alpha_re im + alpha_im re
@@ -331,13 +366,14 @@ __device__ __forceinline__ void sp_store(const GemmArgs& g, const f32x4 (&acc)[G
                         const float y = sp_neighbour(old[i][j][r]), oldoth = odd ? y : -y;
                         v += fmaf(g.beta_re, old[i][j][r], g.beta_im * oldoth);
                     }
-                    if (odd && (g.cflags & ICL_CFLAG_REAL_DIAG) && m == n) v = 0.0f;
+                    if (odd && (g.cflags & ICL_CFLAG_REAL_DIAG) && m_of(i) == nl + 16 * j + r) v = 0.0f;
                 } else {
                     v = beta_zero ? g.alpha_re * acc[i][j][r] : fmaf(g.beta_re, old[i][j][r], g.alpha_re * acc[i][j][r]);
                 }
-                if (CHECK && !tri.keep(m, n)) v = 0.0f;
-                if (on(m, n)) c0[16 * i + (16 * j + r) * cstep] = v;
+                if (CHECK && !CPLX && !keep.has(16 * j + r)) v = 0.0f;
+                if (!CHECK || on.has(16 * j + r)) c0[16 * i + (16 * j + r) * cstep] = v;
             }
+    }
 }
 
 // T in rows of the packed operands: a complex tile has T / 2 rows.
