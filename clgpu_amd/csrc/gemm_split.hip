@@ -46,10 +46,11 @@ constexpr int kGroups = 4; // 16-byte chunks (groups of 8 k) per row, slab and p
 typedef __attribute__((address_space(3))) void sp_lds_void;
 
 // ---------------------------------------------------------------------------
-// Prepass. Packed layout P[slab][plane][k / 8][row][8]: any 64 rows of one (slab,
-// plane, k / 8) are 1 KB of contiguous memory, one LDS DMA instruction, and the LDS
+// Prepass. Packed layout P[slab][row / 64][plane][k / 8][row % 64][8]: 64 rows of one
+// (slab, plane, k / 8) are 1 KB of contiguous memory, one LDS DMA instruction, and the LDS
 // image keeps the rows contiguous (16 bytes apart: fragment reads are free of bank
-// conflicts).
+// conflicts). What a wave copies of a slab lies at constant offsets from one 64-bit
+// address, whatever the number of rows.
 //
 // Complex operands become real ones: op(A) (m x k) the 2m x 2k matrix with the
 // 2 x 2 blocks [re -im; im re], op(B) the 2k x n matrix of its stacked parts, so
@@ -156,12 +157,12 @@ split_pack_kernel(SplitSrc a, SplitSrc b, int ablocks, int slabs, unsigned long 
             out[1][i / 8][i % 8] = lo;
         }
     }
-    __bf16* dst = o.P + (((size_t)ks * PLANES * kGroups + 2 * (w & 1)) * o.Rpad + r0 + r) * 8;
+    __bf16* dst = o.P + ((size_t)ks * o.Rpad + r0) * (PLANES * kGroups * 8) + (2 * (w & 1) * 64 + r) * 8;
 #pragma unroll
     for (int p = 0; p < PLANES; ++p)
 #pragma unroll
         for (int c = 0; c < 2; ++c)
-            *reinterpret_cast<bf16x8*>(dst + (size_t)(kGroups * p + c) * o.Rpad * 8) = out[p][c];
+            *reinterpret_cast<bf16x8*>(dst + (kGroups * p + c) * (64 * 8)) = out[p][c];
 }
 
 // ---------------------------------------------------------------------------
@@ -441,29 +442,25 @@ __global__ void __launch_bounds__(WVM* WVN * 64, T == 256 ? 2 : 4) split_gemm_ke
     const int m0 = tm * T, n0 = tn * T; // packed rows
 
     // This wave's copies of a block: the k groups wave / RB + (NW / RB) i of 64 rows.
-    const size_t a_row = (size_t)p.Mpad * 16, b_row = (size_t)p.Npad * 16; // bytes of one k group of all rows
-    const size_t a_plane = kGroups * a_row, b_plane = kGroups * b_row, a_slab = PLANES * a_plane, b_slab = PLANES * b_plane;
-    const char* a_src = reinterpret_cast<const char*>(p.Ap) + (size_t)ks0 * a_slab + (wave / Cfg::RB) * a_row +
-                        (size_t)(m0 + 64 * (wave % Cfg::RB)) * 16;
-    const char* b_src = reinterpret_cast<const char*>(p.Bp) + (size_t)ks0 * b_slab + (wave / Cfg::RB) * b_row +
-                        (size_t)(n0 + 64 * (wave % Cfg::RB)) * 16;
+    constexpr int ROW_BYTES = PLANES * kGroups * 16; // of one packed row of a slab
+    const size_t a_slab = (size_t)p.Mpad * ROW_BYTES, b_slab = (size_t)p.Npad * ROW_BYTES;
+    const size_t a_row = (size_t)(m0 + 64 * (wave % Cfg::RB)), b_row = (size_t)(n0 + 64 * (wave % Cfg::RB));
+    const char* a_src = reinterpret_cast<const char*>(p.Ap) + ks0 * a_slab + a_row * ROW_BYTES + wave / Cfg::RB * 1024;
+    const char* b_src = reinterpret_cast<const char*>(p.Bp) + ks0 * b_slab + b_row * ROW_BYTES + wave / Cfg::RB * 1024;
     const int loff = lane * 16;
     const int n = ks1 - ks0;
     // Part `i` of the copy of a slab's block c to the ring slot at `slot` (bytes), src
     // being the slab's first byte of op(A) / op(B). A buffer load: its address stays
     // scalar, and a global load would count as a FLAT access, after which the compiler
-    // waits for all LDS reads at once. The plane is part of the 64-bit base and the
-    // descriptor unbounded: a slab of all rows is longer than 32-bit offsets and extents
-    // reach from 2^24 (three planes) or 2^25 rows on. What is left of the offset, 32 bytes
-    // per row, is checked by the launcher.
+    // waits for all LDS reads at once. (A layout with all rows of a plane together reached
+    // past 32-bit offsets and extents from 2^24 rows on.)
     constexpr int PER_SLAB = 2 * PLANES, KSTEP = Cfg::NW / Cfg::RB;
     auto copy = [&](const char* a, const char* b, int c, int slot, int i) {
         const bool of_a = PLANES == 3 ? c >= 3 : (c == 0 || c == 2);
         const int plane = PLANES == 3 ? (c < 3 ? 2 - c : c - 3) : (c == 0 || c == 3 ? 1 : 0);
-        const char* src = of_a ? a + plane * a_plane : b + plane * b_plane;
-        const auto rsrc = __builtin_amdgcn_make_buffer_rsrc(const_cast<char*>(src), 0, 0xffffffffu, 0x20000);
+        const auto rsrc = __builtin_amdgcn_make_buffer_rsrc(const_cast<char*>(of_a ? a : b), 0, 64 * ROW_BYTES, 0x20000);
         __builtin_amdgcn_raw_ptr_buffer_load_lds(rsrc, (sp_lds_void*)(lds_sp + slot + (wave + Cfg::NW * i) * 1024), 16,
-                                                 loff, KSTEP * i * (unsigned)(of_a ? a_row : b_row), 0, 0);
+                                                 loff, (kGroups * plane + KSTEP * i) * 1024, 0, 0);
     };
 
     f32x4 acc[Cfg::FM][Cfg::FN];
@@ -821,12 +818,13 @@ hipError_t sp_product(SplitArgs p, const icl_gemm_args& g, const SplitPlan& plan
                                  (long)plan.rest * (C::NW * C::FM * C::FN / 4), s, p);
 }
 
-// The rows [r0, r0 + rows) of a real source and its packed layout.
+// The rows [r0, r0 + rows) of a real source and its packed layout (r0 a multiple of 64).
+template <int PLANES>
 SplitSrc sp_rows(SplitSrc src, int r0, int rows)
 {
     src.X += src.kcontig ? (long)r0 * src.ld : (long)r0;
     src.R = rows;
-    src.P += (size_t)r0 * 8;
+    src.P += (size_t)r0 * (PLANES * kGroups * 8);
     return src;
 }
 
@@ -836,7 +834,6 @@ hipError_t sp_launch(const icl_gemm_args* g, int opa, int opb, int edge, void* w
     (void)edge;
     if (!ws || (PLANES == 3 && !g->guard)) return hipErrorInvalidValue;
     const SplitLayout l = sp_layout<T, PLANES, CPLX>(g);
-    if (32.0 * std::max(l.Mpad, l.Npad) > UINT_MAX) return hipErrorInvalidValue;
     SplitArgs p{};
     p.Mpad = l.Mpad;
     p.Npad = l.Npad;
@@ -860,10 +857,10 @@ hipError_t sp_launch(const icl_gemm_args* g, int opa, int opb, int edge, void* w
         const icl_side_lane* side = icl_gemm_side_lane();
         const int m0 = sp_round_up(g->M / 2, T), n0 = sp_round_up(g->N / 2, T);
         if (side && !uses_level3(g) && g->M % T == 0 && g->N % T == 0 && m0 < g->M && n0 < g->N) {
-            if ((e = sp_pack<2, false>(sp_rows(a, 0, m0), m0, sp_rows(b, 0, n0), n0, p, s)) != hipSuccess) return e;
+            if ((e = sp_pack<2, false>(sp_rows<2>(a, 0, m0), m0, sp_rows<2>(b, 0, n0), n0, p, s)) != hipSuccess) return e;
             if ((e = hipEventRecord(side->start, s)) != hipSuccess) return e;
             if ((e = hipStreamWaitEvent(side->stream, side->start, 0)) != hipSuccess) return e;
-            e = sp_pack<2, false>(sp_rows(a, m0, g->M - m0), g->M - m0, sp_rows(b, n0, g->N - n0), g->N - n0, p,
+            e = sp_pack<2, false>(sp_rows<2>(a, m0, g->M - m0), g->M - m0, sp_rows<2>(b, n0, g->N - n0), g->N - n0, p,
                                   side->stream);
             if (e != hipSuccess || (e = hipEventRecord(side->done, side->stream)) != hipSuccess) return e;
             if ((e = icl_timer_mark(s)) != hipSuccess) return e;
@@ -876,8 +873,8 @@ hipError_t sp_launch(const icl_gemm_args* g, int opa, int opb, int edge, void* w
                 gq.N = part[q][3];
                 gq.C = g->C + (long)part[q][2] * g->ldc + part[q][0];
                 SplitArgs pq = p;
-                pq.Ap = Ap + (size_t)part[q][0] * 8;
-                pq.Bp = Bp + (size_t)part[q][2] * 8;
+                pq.Ap = Ap + (size_t)part[q][0] * (PLANES * kGroups * 8);
+                pq.Bp = Bp + (size_t)part[q][2] * (PLANES * kGroups * 8);
                 if ((e = sp_product<T, PLANES, CPLX>(pq, gq, SplitPlan{gq.M / T * (gq.N / T), 0, 1, 0.0}, s)) != hipSuccess) return e;
             }
             return icl_timer_mark(s);
