@@ -63,23 +63,31 @@ public:
 
     // Returns at least `bytes` of device memory. Growing waits for `stream` first
     // because queued work may still use the old allocation. Growing beyond the
-    // handle's cap fails like an exhausted device (ALLOC_FAILED), before anything
-    // is freed or allocated.
+    // handle's cap or the device's memory gives up the optional buffer; where that
+    // is not enough for the cap it fails like an exhausted device (ALLOC_FAILED),
+    // before anything is freed or allocated.
     void* get(size_t bytes, hipStream_t stream)
     {
         if (bytes <= cap_ && ptr_) return ptr_;
         const size_t want = bytes < 256 ? 256 : bytes;
-        if (!fits(bytes))
-            throw status_error(ICLBLAS_STATUS_ALLOC_FAILED, "scratch limit of the handle");
+        DeviceScratch* const other = budget_ && budget_->optional != this ? budget_->optional : nullptr;
+        auto give_up = [&] {
+            hip_check(hipStreamSynchronize(stream), "hipStreamSynchronize");
+            other->release();
+        };
+        if (!fits(bytes)) {
+            if (!other || budget_->held - cap_ - other->cap_ + want > budget_->limit)
+                throw status_error(ICLBLAS_STATUS_ALLOC_FAILED, "scratch limit of the handle");
+            give_up();
+        }
         if (ptr_) {
             hip_check(hipStreamSynchronize(stream), "hipStreamSynchronize");
             release();
         }
         hipError_t e = hipMalloc(&ptr_, want);
-        if (e != hipSuccess && budget_ && budget_->optional && budget_->optional != this && budget_->optional->ptr_) {
+        if (e != hipSuccess && other && other->ptr_) {
             (void)hipGetLastError();
-            hip_check(hipStreamSynchronize(stream), "hipStreamSynchronize");
-            budget_->optional->release();
+            give_up();
             e = hipMalloc(&ptr_, want);
         }
         if (e != hipSuccess) ptr_ = nullptr;
