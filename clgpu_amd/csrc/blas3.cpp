@@ -230,6 +230,16 @@ static size_t packed_bytes(int kind, const icl_gemm_args& g)
     return (up(g.M, 128) + up(g.N, 128)) * up(g.K, 32) * (kind == ICL_KIND_CGEMM ? 8 : 4);
 }
 
+// A split-BF16 product without packed operands: on the unpacked kernels, or, as those
+// have no level-3 options, on FP32 MFMA.
+static const icl_gemm_variant* unpacked_variant(GemmProblem& p)
+{
+    p.optional_ws = false;
+    p.no_ws = true;
+    if (level3_problem(*p.args)) p.math = ICL_MATH_FP32;
+    return gemm_best(p);
+}
+
 // A split-BF16 product on a handle with a cap: no partial sums, then the packed
 // implementation that needs the least. A complex one, whose op(A) is packed twice, runs
 // unpacked where the cap admits the operands packed once.
@@ -243,8 +253,7 @@ static const icl_gemm_variant* capped_variant(iclblasContext* h, const icl_gemm_
         for (const icl_gemm_variant* u : gemm_registry())
             if (u->workspace && gemm_accept(*u, p) && u->workspace(&g) < v->workspace(&g)) v = u;
     if (scratch.fits(v->workspace(&g)) || p.kind != ICL_KIND_CGEMM || !scratch.fits(packed_bytes(p.kind, g))) return v;
-    p.no_ws = true;
-    return gemm_best(p);
+    return unpacked_variant(p);
 }
 
 // ---------------------------------------------------------------------------
