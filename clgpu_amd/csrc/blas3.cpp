@@ -223,11 +223,44 @@ static const icl_gemm_variant* gemm_best(const GemmProblem& p)
     return best;
 }
 
-// The packed operands of a split-BF16 product, 4 bytes per element (complex: 8), rounded up to whole 128-row tiles of 32-deep slabs.
-static size_t packed_bytes(int kind, const icl_gemm_args& g)
+// The workspace that a split-BF16 product may insist on, 0 for the ones that run without:
+// what a handle's cap, a captured stream and the static scratch of iclblasSgemmNoAlloc
+// have to have room for. A model of its own, fixed tiles at fixed rates ranked with the
+// unpacked kernels by gemm_score, so that a call is not refused, or a graph does not
+// need memory, because some kernel has become faster. The operands are packed once, 4
+// bytes per element (complex: 8).
+template <int BM, int BN, int BK, int BYTES>
+static size_t packed_once(const icl_gemm_args* g)
 {
     auto up = [](int x, int m) { return (size_t)((x + m - 1) / m) * m; };
-    return (up(g.M, 128) + up(g.N, 128)) * up(g.K, 32) * (kind == ICL_KIND_CGEMM ? 8 : 4);
+    return (up(g->M, BM) + up(g->N, BN)) * up(g->K, BK) * BYTES;
+}
+#define ICL_PACKED_TILE(kind, BM, BN, BK, THREADS, BYTES, TF, OCC)                                                     \
+    {"", kind, ICL_MATH_BF16X3, BM, BN, BK, THREADS, nullptr, packed_once<BM, BN, BK, BYTES>, TF, OCC, 1, nullptr}
+static const icl_gemm_variant kPackedTiles[] = {
+    ICL_PACKED_TILE(ICL_KIND_SGEMM, 256, 256, 32, 512, 4, 463.0f, 1),
+    ICL_PACKED_TILE(ICL_KIND_SGEMM, 128, 128, 32, 256, 4, 366.0f, 2),
+    ICL_PACKED_TILE(ICL_KIND_CGEMM, 256, 128, 16, 512, 8, 495.0f, 1),
+    ICL_PACKED_TILE(ICL_KIND_CGEMM, 128, 128, 16, 256, 8, 387.0f, 1),
+};
+#undef ICL_PACKED_TILE
+
+size_t gemm_required_workspace(const GemmProblem& p)
+{
+    const icl_gemm_variant* best = nullptr;
+    float best_score = -1.0f;
+    auto rank = [&](const icl_gemm_variant* v) {
+        if (!gemm_accept(*v, p)) return;
+        const float s = gemm_score(*v, p);
+        if (s > best_score) {
+            best = v;
+            best_score = s;
+        }
+    };
+    for (const icl_gemm_variant* v : gemm_registry())
+        if (!v->workspace) rank(v);
+    for (const icl_gemm_variant& v : kPackedTiles) rank(&v);
+    return best && best->workspace ? best->workspace(p.args) : 0;
 }
 
 // A split-BF16 product without packed operands: on the unpacked kernels, or, as those
@@ -240,22 +273,6 @@ static const icl_gemm_variant* unpacked_variant(GemmProblem& p)
     return gemm_best(p);
 }
 
-// A split-BF16 product on a handle with a cap: no partial sums, then the packed
-// implementation that needs the least. A complex one, whose op(A) is packed twice, runs
-// unpacked where the cap admits the operands packed once.
-static const icl_gemm_variant* capped_variant(iclblasContext* h, const icl_gemm_variant* v, GemmProblem& p,
-                                              icl_gemm_args& g)
-{
-    const icl::DeviceScratch& scratch = h->scratch[iclblasContext::kSlotGemmWorkspace];
-    g.whole_depth = 1;
-    if (scratch.fits(v->workspace(&g))) return v;
-    if (h->forced_impl.empty())
-        for (const icl_gemm_variant* u : gemm_registry())
-            if (u->workspace && gemm_accept(*u, p) && u->workspace(&g) < v->workspace(&g)) v = u;
-    if (scratch.fits(v->workspace(&g)) || p.kind != ICL_KIND_CGEMM || !scratch.fits(packed_bytes(p.kind, g))) return v;
-    return unpacked_variant(p);
-}
-
 // ---------------------------------------------------------------------------
 // GEMM
 // ---------------------------------------------------------------------------
@@ -265,17 +282,81 @@ static const icl_gemm_variant* capped_variant(iclblasContext* h, const icl_gemm_
 // 3 k 2^-24 |a||b| once k >= 256. Smaller K runs on FP32 MFMA instead.
 constexpr int kSplitMinK = 256;
 
+static bool capturing(hipStream_t s)
+{
+    hipStreamCaptureStatus capture = hipStreamCaptureStatusNone;
+    hip_check(hipStreamIsCapturing(s, &capture), "hipStreamIsCapturing");
+    return capture != hipStreamCaptureStatusNone;
+}
+
 // Whether a product may use memory that only makes it faster: not when it could not
 // pay, when the caller has capped the handle's memory or forbidden allocation, and
 // not while the stream is being captured (a later call could free a workspace that
 // the graph would use).
-static bool optional_workspace(iclblasContext* h, int kind, const icl_gemm_args& g, hipStream_t s)
+static bool optional_workspace(iclblasContext* h, int kind, int math, const icl_gemm_args& g, hipStream_t s)
 {
     if (g.K <= 0 || h->ext_ws || h->budget.limit || s != h->stream) return false;
-    if (h->forced_impl.empty() && !split3_candidate(kind, g)) return false;
-    hipStreamCaptureStatus capture = hipStreamCaptureStatusNone;
-    hip_check(hipStreamIsCapturing(s, &capture), "hipStreamIsCapturing");
-    return capture == hipStreamCaptureStatusNone;
+    if (math == ICL_MATH_FP32 && h->forced_impl.empty() && !split3_candidate(kind, g)) return false;
+    return !capturing(s);
+}
+
+// Whether a packed split-BF16 product fits in `room` bytes, and then how: with partial
+// sums (unless whole), over its whole depth, or on the packed variant that needs least.
+static bool fit_packed(iclblasContext* h, const icl_gemm_variant*& v, const GemmProblem& p, icl_gemm_args& g,
+                       size_t room, bool whole)
+{
+    g.whole_depth = whole;
+    if (v->workspace(&g) <= room) return true;
+    g.whole_depth = 1;
+    if (v->workspace(&g) <= room) return true;
+    if (h->forced_impl == v->name) return false;
+    for (const icl_gemm_variant* u : gemm_registry())
+        if (u->workspace && gemm_accept(*u, p) && u->workspace(&g) <= room) {
+            v = u;
+            return true;
+        }
+    return false;
+}
+
+// The workspace of a split-BF16 product that gemm_select gave the packed variant v; may
+// replace v by one that needs less, or none. Under a cap, in a captured stream and with
+// the caller's scratch the product is refused when what it requires cannot be had, and
+// takes no more than that, except into the optional buffer. A complex product needs more
+// than its operands packed once (op(A) is packed as rows of two parts): without room for
+// that it runs unpacked.
+static void* packed_workspace(iclblasContext* h, const icl_gemm_variant*& v, GemmProblem& p, icl_gemm_args& g,
+                              hipStream_t s)
+{
+    icl::DeviceScratch& own = h->scratch[iclblasContext::kSlotGemmWorkspace];
+    icl::DeviceScratch& spare = h->scratch[iclblasContext::kSlotSplit3];
+    const bool forced = h->forced_impl == v->name;
+    if (p.optional_ws) {
+        if (void* ws = own.try_get(v->workspace(&g), s)) return ws;
+        p.optional_ws = false;
+    }
+    icl_gemm_args once = g;
+    once.whole_depth = 1;
+    const size_t required = forced ? v->workspace(&once) : gemm_required_workspace(p);
+    if (required == 0) {
+        v = unpacked_variant(p);
+        return nullptr;
+    }
+    if (h->ext_ws) {
+        if (required > h->ext_ws_bytes || !fit_packed(h, v, p, g, h->ext_ws_bytes, false))
+            throw status_error(ICLBLAS_STATUS_INVALID_VALUE, "GEMM workspace exceeds the caller's scratch");
+        return h->ext_ws;
+    }
+    const bool capped = h->budget.limit != 0;
+    if (fit_packed(h, v, p, g, own.capacity(), capped)) return own.get(v->workspace(&g), s);
+    if (p.kind == ICL_KIND_SGEMM || forced) {
+        (void)fit_packed(h, v, p, g, required, true);
+        return own.get(required, s);
+    }
+    if (!own.fits(required, true)) throw status_error(ICLBLAS_STATUS_ALLOC_FAILED, "scratch limit of the handle");
+    if (capped && !capturing(s) && fit_packed(h, v, p, g, spare.room(), true))
+        if (void* ws = spare.try_get(v->workspace(&g), s)) return ws;
+    v = unpacked_variant(p);
+    return nullptr;
 }
 
 // The product on a three-way split kernel `v`, then the FP32 MFMA kernel `native`
@@ -307,7 +388,7 @@ static void run_gemm(iclblasContext* h, int kind, int math, int opa, int opb, ic
     if (math == ICL_MATH_BF16X3 && g.K < kSplitMinK) math = ICL_MATH_FP32;
     const hipStream_t s = stream ? stream : h->stream;
     GemmProblem p{kind, math, opa, opb, &g};
-    p.optional_ws = optional_workspace(h, kind, g, s);
+    p.optional_ws = optional_workspace(h, kind, math, g, s);
     const icl_gemm_variant* v = gemm_select(h, p);
     if (level3_problem(g) && !v->level3)
         throw status_error(ICLBLAS_STATUS_INTERNAL_ERROR, "level-3 GEMM options on a kernel without them");
@@ -320,25 +401,7 @@ static void run_gemm(iclblasContext* h, int kind, int math, int opa, int opb, ic
         }
         v = native;
     }
-    if (v->workspace && h->budget.limit && !h->ext_ws) v = capped_variant(h, v, p, g);
-    void* ws = nullptr;
-    if (v->workspace) {
-        if (h->ext_ws && v->workspace(&g) > h->ext_ws_bytes) g.whole_depth = 1;
-        const size_t bytes = v->workspace(&g);
-        if (bytes && h->ext_ws) {
-            if (bytes > h->ext_ws_bytes)
-                throw status_error(ICLBLAS_STATUS_INVALID_VALUE, "GEMM workspace exceeds the caller's scratch");
-            ws = h->ext_ws;
-        } else if (bytes) {
-            icl::DeviceScratch& scratch = h->scratch[iclblasContext::kSlotGemmWorkspace];
-            if (p.optional_ws) ws = scratch.try_get(bytes, h->stream);
-            if (!ws) {
-                p.optional_ws = false; // the implementation that needs no more than it must
-                v = h->forced_impl.empty() && !h->budget.limit ? gemm_best(p) : v;
-                if (v->workspace) ws = scratch.get(v->workspace(&g), h->stream);
-            }
-        }
-    }
+    void* ws = v->workspace ? packed_workspace(h, v, p, g, s) : nullptr;
     const bool edge = gemm_needs_edge(*v, p);
     // A variant with a prepass marks its main kernel itself (icl_timer_mark),
     // and may run half of the prepass on the handle's side stream: offered for
@@ -430,7 +493,7 @@ static bool band_split_pays(iclblasContext* h, int kind, int math, int opa, int 
         return false;
     {
         GemmProblem whole{kind, math, opa, opb, &g};
-        whole.optional_ws = optional_workspace(h, kind, g, h->stream);
+        whole.optional_ws = optional_workspace(h, kind, math, g, h->stream);
         if (gemm_select(h, whole)->workspace) return false;
     }
     auto est = [&](int tri) {

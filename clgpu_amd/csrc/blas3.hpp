@@ -35,6 +35,9 @@ bool gemm_needs_edge(const icl_gemm_variant& v, const GemmProblem& p);
 // this kind. Throws NOT_SUPPORTED when nothing accepts.
 const icl_gemm_variant* gemm_select(iclblasContext* h, const GemmProblem& p);
 
+// Bytes of workspace that a split-BF16 product may require of its caller (0: none).
+size_t gemm_required_workspace(const GemmProblem& p);
+
 // ---- algorithms ----
 // C = alpha*op(A)*op(B) + beta*C (real). mask: ICL_MASK_* applied to the stored C.
 void sgemm_dev(iclblasContext* h, int math, int opa, int opb, int m, int n, int k, float alpha, const float* A,

@@ -9,6 +9,8 @@
 #pragma once
 #include <hip/hip_runtime_api.h>
 
+#include <algorithm>
+#include <cstdint>
 #include <mutex>
 #include <stdexcept>
 #include <string>
@@ -54,11 +56,20 @@ public:
 
     void set_budget(ScratchBudget* b) { budget_ = b; }
 
-    // Whether get(bytes) stays within the handle's cap.
-    bool fits(size_t bytes) const
+    size_t capacity() const { return cap_; }
+
+    // Bytes that get() gives within the handle's cap; giving_up: or without the
+    // optional buffer.
+    size_t room(bool giving_up = false) const
     {
-        const size_t want = bytes < 256 ? 256 : bytes;
-        return (ptr_ && bytes <= cap_) || !budget_ || !budget_->limit || budget_->held - cap_ + want <= budget_->limit;
+        if (!budget_ || !budget_->limit) return SIZE_MAX;
+        const DeviceScratch* o = giving_up ? budget_->optional : nullptr;
+        const size_t others = budget_->held - cap_ - (o && o != this ? o->cap_ : 0);
+        return std::max(cap_, budget_->limit > others ? budget_->limit - others : 0);
+    }
+    bool fits(size_t bytes, bool giving_up = false) const
+    {
+        return (ptr_ && bytes <= cap_) || std::max(bytes, size_t(256)) <= room(giving_up);
     }
 
     // Returns at least `bytes` of device memory. Growing waits for `stream` first
@@ -76,8 +87,7 @@ public:
             other->release();
         };
         if (!fits(bytes)) {
-            if (!other || budget_->held - cap_ - other->cap_ + want > budget_->limit)
-                throw status_error(ICLBLAS_STATUS_ALLOC_FAILED, "scratch limit of the handle");
+            if (!fits(bytes, true)) throw status_error(ICLBLAS_STATUS_ALLOC_FAILED, "scratch limit of the handle");
             give_up();
         }
         if (ptr_) {
@@ -98,10 +108,11 @@ public:
     }
 
     // The same for memory that only makes a call faster: nullptr instead of an
-    // error when the device has none left.
+    // error when the cap or the device has none left.
     void* try_get(size_t bytes, hipStream_t stream)
     {
         if (bytes <= cap_ && ptr_) return ptr_;
+        if (!fits(bytes)) return nullptr;
         if (ptr_) {
             hip_check(hipStreamSynchronize(stream), "hipStreamSynchronize");
             release();

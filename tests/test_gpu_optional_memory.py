@@ -92,3 +92,83 @@ def test_complex_level3_under_a_cap(routine, v, shape, packed_once):
     assert np.all((err <= bound)[written])
     assert np.array_equal(C[:rc, :cc][~written], c["C"][:rc, :cc][~written])
     torch.cuda.synchronize()
+
+
+def _split_product(h, cplx, m, n, k, call=None):
+    """A product in the split-BF16 mode on device memory: (status, check of the result)."""
+    import torch
+    gen = torch.Generator("cuda").manual_seed(13)
+    dt = torch.complex64 if cplx else torch.float32
+    A, B = (torch.rand(s, device="cuda", generator=gen, dtype=dt) - 0.5 for s in ((k, m), (n, k)))
+    C = torch.full((n, m), float("nan"), device="cuda", dtype=dt)
+    torch.cuda.synchronize()
+    call = call or (ib.iclblasCgemm if cplx else ib.iclblasSgemm)
+
+    def run():
+        return call(h.value, 0, 0, m, n, k, 1.0, A.data_ptr(), m, B.data_ptr(), k, 0.0, C.data_ptr(), m)
+
+    def check():
+        wide = torch.complex128 if cplx else torch.float64
+        err = (C.to(wide) - B.to(wide) @ A.to(wide)).abs()
+        kk = 2 * k if cplx else k
+        assert bool((err <= 4 * kk * U32 * (2 if cplx else 1) * (B.abs().double() @ A.abs().double())).all())
+    return run, check, C
+
+
+# (complex, m, n, k, bytes): what a split-BF16 product requires is part of the library's behaviour under
+# a cap. Operands packed once, rows in tiles of 128 or 256, or nothing: several of the latter run on the
+# packed kernels where memory is free.
+REQUIRED = [(False, 1024, 1024, 1024, 8388608), (False, 700, 900, 300, 2293760), (False, 1280, 2944, 1280, 21626880),
+            (False, 130, 4000, 3000, 52363264), (True, 640, 700, 512, 0), (True, 1030, 1111, 300, 0),
+            (True, 1664, 512, 641, 0), (True, 2304, 2048, 335, 0), (True, 1500, 1400, 1300, 30900224),
+            (True, 129, 3000, 2000, 0)]
+
+
+@pytest.mark.parametrize("cplx,m,n,k,required", REQUIRED)
+def test_required_workspace_under_a_cap(cplx, m, n, k, required):
+    import torch
+    if required:
+        with _handle(ib.MATH_SPLIT_BF16X3) as h:
+            run, _, C = _split_product(h, cplx, m, n, k)
+            h.set_scratch_limit(required - 1)
+            assert run() == ib.STATUS_ALLOC_FAILED
+            h.synchronize()
+            assert bool(torch.isnan(C).all())
+    for cap in (max(required, 256), 3 * required + (64 << 10)):
+        with _handle(ib.MATH_SPLIT_BF16X3) as h:
+            run, check, _ = _split_product(h, cplx, m, n, k)
+            h.set_scratch_limit(cap)
+            ib.check(run())
+            h.synchronize()
+            check()
+            assert "bf16x3" in h.last_implementation() and h.scratch_usage()[0] <= cap
+
+
+@pytest.mark.parametrize("m,n,k", [(2304, 2048, 335), (1664, 512, 641)])
+def test_captured_product_that_requires_nothing(m, n, k):
+    """Captured without a call before it on that handle: it may not allocate."""
+    import torch
+    side = torch.cuda.Stream()
+    with _handle(ib.MATH_SPLIT_BF16X3, side) as h:
+        run, check, C = _split_product(h, True, m, n, k)
+        graph = torch.cuda.CUDAGraph()
+        with torch.cuda.graph(graph, stream=side):
+            ib.check(run())
+        assert h.scratch_usage()[0] == 0
+        for _ in range(3):
+            C.fill_(float("nan"))
+            torch.cuda.synchronize()
+            graph.replay()
+            torch.cuda.synchronize()
+            check()
+
+
+def test_no_alloc_takes_the_variant_that_fits():
+    """4608 x 2944 x 2208: 63.6 MiB of packed operands in rows of 128, 64.7 in rows of 256."""
+    m, n, k = 4608, 2944, 2208
+    with _handle(ib.MATH_SPLIT_BF16X3) as h:
+        run, check, _ = _split_product(h, False, m, n, k, ib.iclblasSgemmNoAlloc)
+        ib.check(run())
+        h.synchronize()
+        check()
+        assert h.last_implementation().startswith("sgemm_bf16x3d") and h.scratch_usage()[0] == 0
