@@ -330,13 +330,17 @@ static void* packed_workspace(iclblasContext* h, const icl_gemm_variant*& v, Gem
     icl::DeviceScratch& own = h->scratch[iclblasContext::kSlotGemmWorkspace];
     icl::DeviceScratch& spare = h->scratch[iclblasContext::kSlotSplit3];
     const bool forced = h->forced_impl == v->name;
-    if (p.optional_ws) {
-        if (void* ws = own.try_get(v->workspace(&g), s)) return ws;
-        p.optional_ws = false;
-    }
     icl_gemm_args once = g;
     once.whole_depth = 1;
     const size_t required = forced ? v->workspace(&once) : gemm_required_workspace(p);
+    if (p.optional_ws) {
+        // The lasting buffer grows, which frees the old one under any graph that holds it,
+        // only for what a product requires: more goes to the optional buffer.
+        const size_t bytes = v->workspace(&g);
+        const bool lasting = bytes <= own.capacity() || required > own.capacity();
+        if (void* ws = (lasting ? own : spare).try_get(bytes, s)) return ws;
+        p.optional_ws = false;
+    }
     if (required == 0) {
         v = unpacked_variant(p);
         return nullptr;

@@ -172,3 +172,40 @@ def test_no_alloc_takes_the_variant_that_fits():
         h.synchronize()
         check()
         assert h.last_implementation().startswith("sgemm_bf16x3d") and h.scratch_usage()[0] == 0
+
+
+def test_a_graph_keeps_its_workspace():
+    """A captured product, then one that requires no more but would like partial sums: its larger workspace
+    is not the one that the graph holds."""
+    import torch
+    side = torch.cuda.Stream()
+    with _handle(ib.MATH_SPLIT_BF16X3, side) as h:
+        run, check, C = _split_product(h, False, 4096, 4096, 1024)  # packed: 32 MiB
+        ib.check(run())
+        h.synchronize()
+        held = h.scratch_usage()[0]
+        assert held == 32 << 20
+        graph = torch.cuda.CUDAGraph()
+        with torch.cuda.graph(graph, stream=side):
+            ib.check(run())
+        with _handle(ib.MATH_SPLIT_BF16X3) as other:
+            ib.check(_split_product(other, False, 1024, 1024, 4096)[0]())
+            other.synchronize()
+            more = other.scratch_usage()[0]
+        assert more > held  # packed: 32 MiB, and partial sums
+        run2, check2, _ = _split_product(h, False, 1024, 1024, 4096)
+        ib.check(run2())
+        h.synchronize()
+        assert h.scratch_usage()[0] == held + more
+        check2()
+        fill = torch.full((64 << 20,), float("nan"), device="cuda")
+        for _ in range(3):
+            C.fill_(float("nan"))
+            torch.cuda.synchronize()
+            graph.replay()
+            torch.cuda.synchronize()
+            check()
+            ib.check(run2())
+            h.synchronize()
+            check2()
+        del fill
