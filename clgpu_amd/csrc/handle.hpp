@@ -37,6 +37,17 @@ inline void hip_check(hipError_t e, const char* what)
     throw status_error(ICLBLAS_STATUS_EXECUTION_FAILED, std::string(what) + ": " + hipGetErrorString(e));
 }
 
+// While it lives, this thread may allocate although some other stream is being captured
+// in the global mode: hipMalloc would fail and invalidate that capture.
+class RelaxedCapture {
+public:
+    RelaxedCapture() { hip_check(hipThreadExchangeStreamCaptureMode(&mode_), "hipThreadExchangeStreamCaptureMode"); }
+    ~RelaxedCapture() { (void)hipThreadExchangeStreamCaptureMode(&mode_); }
+
+private:
+    hipStreamCaptureMode mode_ = hipStreamCaptureModeRelaxed;
+};
+
 // Device memory held by a handle's scratch buffers, and its cap
 // (iclblasSetScratchLimit; 0 = none).
 class DeviceScratch;
@@ -108,11 +119,13 @@ public:
     }
 
     // The same for memory that only makes a call faster: nullptr instead of an
-    // error when the cap or the device has none left.
+    // error when the cap or the device has none left. A call that could do without
+    // does not disturb another stream's capture for it.
     void* try_get(size_t bytes, hipStream_t stream)
     {
         if (bytes <= cap_ && ptr_) return ptr_;
         if (!fits(bytes)) return nullptr;
+        RelaxedCapture relaxed;
         if (ptr_) {
             hip_check(hipStreamSynchronize(stream), "hipStreamSynchronize");
             release();

@@ -209,3 +209,31 @@ def test_a_graph_keeps_its_workspace():
             h.synchronize()
             check2()
         del fill
+
+
+def test_optional_memory_leaves_a_capture_alone():
+    """FP32 products on a stream of their own while another stream is captured: they take their optional
+    workspace, the second a larger one, and the capture stays valid."""
+    import torch
+    n = 2048
+    tA, tB, tC, tD = (torch.rand((2 * n, n), device="cuda") for _ in range(4))
+    x = torch.zeros(1024, device="cuda")
+    captured, other = torch.cuda.Stream(), torch.cuda.Stream()
+    torch.cuda.synchronize()
+    with _handle(stream=other) as h:
+        graph = torch.cuda.CUDAGraph()
+        with torch.cuda.graph(graph, stream=captured):
+            x += 1
+            _sgemm(h, n, tA, tB, tC)
+            assert "split3" in h.last_implementation()
+            held = h.scratch_usage()[0]
+            _sgemm(h, n, tA, tB, tD, m=2 * n)
+            assert h.scratch_usage()[0] > held > 0
+            x += 1
+        h.synchronize()
+        for i in range(3):
+            graph.replay()
+            torch.cuda.synchronize()
+            assert bool((x == 2 * (i + 1)).all())
+    E = (tB[:n].double() @ tA[:n].double())
+    assert bool(((tC[:n] - E).abs() <= 4 * n * U32 * E).all())
