@@ -795,6 +795,7 @@ double sp_estimate(const icl_gemm_args* g)
 template <int PLANES, bool CPLX>
 hipError_t sp_pack(const SplitSrc& a, int arows, const SplitSrc& b, int brows, const SplitArgs& p, hipStream_t s)
 {
+    if (p.slabs == 0) return hipSuccess; // C is only scaled
     const unsigned deep = (unsigned)((p.slabs + 1) / 2), layer = std::min(deep, 32768u);
     const dim3 grid((unsigned)((arows + brows) / 64), layer, (deep + layer - 1) / layer);
     hipLaunchKernelGGL((split_pack_kernel<PLANES, CPLX>), grid, dim3(256), 0, s, a, b, arows / 64, p.slabs,

@@ -21,12 +21,12 @@ constexpr int kWvWaves = 8;
 
 typedef float f32x4_any __attribute__((ext_vector_type(4), aligned(4)));
 
-// One lane's part of a block: row `x` (already at the lane's row), the k from k0 on that
-// this half of the wave takes, zeros from K on. KC: k contiguous, else stride ld.
 // Floats of one operand per lane and block: a block's products take 1024 cycles.
 template <bool CPLX>
 constexpr int kWvVals = CPLX ? 8 : 16;
 
+// One lane's part of a block: row `x` (already at the lane's row), the k from k0 on that
+// this half of the wave takes, zeros from K on. KC: k contiguous, else stride ld.
 template <bool CPLX, bool KC>
 struct WaveOperand {
     const float* x;
@@ -176,7 +176,6 @@ __global__ void __launch_bounds__(kWvWaves * 64, 4) wave_gemm_kernel(GemmArgs g,
 
 namespace {
 
-
 template <bool CPLX, bool A_KC, bool B_KC>
 hipError_t wave_run(const icl_gemm_args* g, int opa, int opb, hipStream_t s)
 {
@@ -191,7 +190,6 @@ hipError_t wave_run(const icl_gemm_args* g, int opa, int opb, hipStream_t s)
 template <bool CPLX>
 hipError_t wave_launch(const icl_gemm_args* g, int opa, int opb, int, void*, hipStream_t s)
 {
-    if (g->K <= 0) return hipErrorInvalidValue;
     if (opa) return opb ? wave_run<CPLX, true, false>(g, opa, opb, s) : wave_run<CPLX, true, true>(g, opa, opb, s);
     return opb ? wave_run<CPLX, false, false>(g, opa, opb, s) : wave_run<CPLX, false, true>(g, opa, opb, s);
 }
