@@ -172,14 +172,14 @@ static const icl_gemm_variant* gemm_best(const GemmProblem& p)
     double split_time = 0.0;
     const bool splits = p.optional_ws && split3_candidate(p.kind, *p.args);
     for (const icl_gemm_variant* v : gemm_registry()) {
-        if (!gemm_accept(*v, p) || (p.no_ws && v->workspace)) continue;
+        if (!gemm_accept(*v, p) || (p.no_ws && v->workspace) || (p.tiled && (v->workspace || v->estimate))) continue;
         if (!v->workspace && v->estimate) {
             wave = v;
             continue;
         }
-        if (v->workspace && splits && v->workspace(p.args) <= kSplit3MaxBytes) {
+        if (v->workspace && splits) {
             const double t = v->estimate(p.args);
-            if (!split || t < split_time) {
+            if ((!split || t < split_time) && v->workspace(p.args) <= kSplit3MaxBytes) {
                 split = v;
                 split_time = t;
             }
@@ -199,9 +199,9 @@ static const icl_gemm_variant* gemm_best(const GemmProblem& p)
         // (1024 x 1536 x 1024: 49 us against 40). Chosen so, 120 random products lost 1%
         // against the fastest kernel of each (all on FP32 MFMA tiles: 50%).
         double t = tiled_time(p, *best);
-        if (wave && wave->estimate(p.args) < 0.9 * t) {
+        if (const double w = wave ? wave->estimate(p.args) : t; w < 0.9 * t) {
             best = wave;
-            t = wave->estimate(p.args);
+            t = w;
         }
         const double margin = best->math == ICL_MATH_FP32 && p.kind == ICL_KIND_SGEMM && real_macs(p.kind, *p.args) < 2e9 ? 1.33
                               : p.args->write_tri != ICL_TRI_NONE ? 1.25 // tiled_time is high for short triangles
@@ -387,12 +387,13 @@ static bool run_split3(iclblasContext* h, const icl_gemm_variant* v, const icl_g
 // `stream`: the stream to run on (default the handle's; a variant with a
 // workspace always runs on the handle's stream).
 static void run_gemm(iclblasContext* h, int kind, int math, int opa, int opb, icl_gemm_args g, bool record,
-                     hipStream_t stream = nullptr)
+                     hipStream_t stream = nullptr, bool tiled = false)
 {
     if (math == ICL_MATH_BF16X3 && g.K < kSplitMinK) math = ICL_MATH_FP32;
     const hipStream_t s = stream ? stream : h->stream;
     GemmProblem p{kind, math, opa, opb, &g};
-    p.optional_ws = optional_workspace(h, kind, math, g, s);
+    p.tiled = tiled;
+    p.optional_ws = !tiled && optional_workspace(h, kind, math, g, s);
     const icl_gemm_variant* v = gemm_select(h, p);
     if (level3_problem(g) && !v->level3)
         throw status_error(ICLBLAS_STATUS_INTERNAL_ERROR, "level-3 GEMM options on a kernel without them");
@@ -495,18 +496,19 @@ static bool band_split_pays(iclblasContext* h, int kind, int math, int opa, int 
     if (!h->forced_impl.empty() || math != ICL_MATH_FP32 || g.kband != ICL_KBAND_NONE || g.M != g.N ||
         g.M < 2 * ICL_TRI_BAND_BLOCK || (g.write_tri != ICL_TRI_LOWER && g.write_tri != ICL_TRI_UPPER))
         return false;
-    {
-        GemmProblem whole{kind, math, opa, opb, &g};
-        whole.optional_ws = optional_workspace(h, kind, math, g, h->stream);
-        if (gemm_select(h, whole)->workspace) return false;
-    }
     auto est = [&](int tri) {
         icl_gemm_args t = g;
         t.write_tri = tri;
-        const GemmProblem p{kind, math, opa, opb, &t};
-        return 1.0 / gemm_score(*gemm_select(h, p), p);
+        GemmProblem p{kind, math, opa, opb, &t};
+        p.tiled = true;
+        return 1.0 / gemm_score(*gemm_best(p), p);
     };
-    return est(g.write_tri | ICL_TRI_OFF_BAND) + est(g.write_tri | ICL_TRI_BAND) < 0.97 * est(g.write_tri);
+    if (est(g.write_tri | ICL_TRI_OFF_BAND) + est(g.write_tri | ICL_TRI_BAND) >= 0.97 * est(g.write_tri)) return false;
+    // The pair is two of the tiled launches that the model ranks; the packed and the wave
+    // kernels run the triangle whole.
+    GemmProblem whole{kind, math, opa, opb, &g};
+    whole.optional_ws = optional_workspace(h, kind, math, g, h->stream);
+    return !gemm_best(whole)->estimate;
 }
 
 void gemm_level3_dev(iclblasContext* h, int kind, int opa, int opb, int m, int n, int k, const float alpha[2],
@@ -543,20 +545,20 @@ void gemm_level3_dev(iclblasContext* h, int kind, int opa, int opb, int m, int n
         const icl_side_lane* side = h->side.ensure();
         hip_check(hipEventRecord(side->start, h->stream), "hipEventRecord");
         g.write_tri = write_tri | ICL_TRI_OFF_BAND;
-        run_gemm(h, kind, math, opa, opb, g, true);
+        run_gemm(h, kind, math, opa, opb, g, true, nullptr, true);
         hip_check(hipStreamWaitEvent(side->stream, side->start, 0), "hipStreamWaitEvent");
         g.write_tri = write_tri | ICL_TRI_BAND;
-        run_gemm(h, kind, math, opa, opb, g, true, side->stream);
+        run_gemm(h, kind, math, opa, opb, g, true, side->stream, true);
         hip_check(hipEventRecord(side->done, side->stream), "hipEventRecord");
         hip_check(hipStreamWaitEvent(h->stream, side->done, 0), "hipStreamWaitEvent");
         return;
     }
     if (split) {
         g.write_tri = write_tri | ICL_TRI_OFF_BAND;
-        run_gemm(h, kind, math, opa, opb, g, true);
+        run_gemm(h, kind, math, opa, opb, g, true, nullptr, true);
         g.write_tri = write_tri | ICL_TRI_BAND;
     }
-    run_gemm(h, kind, math, opa, opb, g, true);
+    run_gemm(h, kind, math, opa, opb, g, true, nullptr, split);
 }
 
 // ---------------------------------------------------------------------------

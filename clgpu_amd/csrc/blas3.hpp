@@ -18,6 +18,7 @@ struct GemmProblem {
     const icl_gemm_args* args;
     bool optional_ws = false; // FP32 implementations that need a workspace are candidates
     bool no_ws = false;       // no implementation that needs a workspace is one
+    bool tiled = false;       // only those are that gemm_score ranks: neither packed nor wave kernels
 };
 
 // Every registered GEMM implementation, in registration order.

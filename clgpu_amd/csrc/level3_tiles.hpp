@@ -37,10 +37,19 @@ __host__ __device__ __attribute__((always_inline)) inline void tri_tile_row(int 
     cnt = b > a ? b - a : 0;
 }
 
-// Number of tiles of an M x N output that meet the written triangle.
+// Number of tiles of an M x N output that meet the written triangle. Square tiles, most
+// of those that a call's choice of implementation asks about a dozen times, are counted
+// in closed form (3008 x 3008, a choice: 0.79 us row by row, 0.33).
 __host__ __device__ inline long tri_tile_count(int M, int N, int write_tri, int bm, int bn)
 {
     const int tiles_m = (M + bm - 1) / bm, tiles_n = (N + bn - 1) / bn;
+    const long t = tiles_m < tiles_n ? tiles_m : tiles_n;
+    if (bm == bn && (write_tri & 12) == 0)
+        return (write_tri & 3) == 1 ? t * (t + 1) / 2 + (tiles_m - t) * tiles_n : t * tiles_n - t * (t - 1) / 2;
+    if (bm == bn && tiles_m == tiles_n) {
+        const long q = 256 / bm, r = t % q, on_blocks = t / q * (q * (q + 1) / 2) + r * (r + 1) / 2;
+        return (write_tri & 8) ? on_blocks : t * (t + 1) / 2 - on_blocks;
+    }
     long total = 0;
     for (int tm = 0; tm < tiles_m; ++tm) {
         int lo, cnt;
