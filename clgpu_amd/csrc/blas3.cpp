@@ -300,22 +300,27 @@ static bool optional_workspace(iclblasContext* h, int kind, int math, const icl_
     return !capturing(s);
 }
 
-// Whether a packed split-BF16 product fits in `room` bytes, and then how: with partial
-// sums (unless whole), over its whole depth, or on the packed variant that needs least.
+// Whether a packed split-BF16 product fits in `room` bytes, and then how: the variant, and
+// partial sums (unless whole) or the whole depth, that estimate the shortest time there.
 static bool fit_packed(iclblasContext* h, const icl_gemm_variant*& v, const GemmProblem& p, icl_gemm_args& g,
                        size_t room, bool whole)
 {
-    g.whole_depth = whole;
-    if (v->workspace(&g) <= room) return true;
-    g.whole_depth = 1;
-    if (v->workspace(&g) <= room) return true;
-    if (h->forced_impl == v->name) return false;
-    for (const icl_gemm_variant* u : gemm_registry())
-        if (u->workspace && gemm_accept(*u, p) && u->workspace(&g) <= room) {
-            v = u;
-            return true;
+    const bool forced = h->forced_impl == v->name;
+    const icl_gemm_variant* best = nullptr;
+    int best_whole = 1;
+    double best_time = 0.0;
+    for (g.whole_depth = whole; g.whole_depth <= 1; ++g.whole_depth)
+        for (const icl_gemm_variant* u : gemm_registry()) {
+            if (forced ? u != v : !u->workspace || !gemm_accept(*u, p)) continue;
+            const double t = u->estimate(&g);
+            if ((best && t >= best_time) || u->workspace(&g) > room) continue;
+            best = u;
+            best_whole = g.whole_depth;
+            best_time = t;
         }
-    return false;
+    g.whole_depth = best_whole;
+    if (best) v = best;
+    return best != nullptr;
 }
 
 // The workspace of a split-BF16 product that gemm_select gave the packed variant v; may
