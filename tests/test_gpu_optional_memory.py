@@ -237,3 +237,15 @@ def test_optional_memory_leaves_a_capture_alone():
             assert bool((x == 2 * (i + 1)).all())
     E = (tB[:n].double() @ tA[:n].double())
     assert bool(((tC[:n] - E).abs() <= 4 * n * U32 * E).all())
+
+
+def test_no_alloc_in_the_fp32_mode():
+    """Where iclblasSgemm takes the packed kernels: FP32 MFMA, no memory, a result within the same bound."""
+    for call, name in ((ib.iclblasSgemm, "split3"), (ib.iclblasSgemmNoAlloc, "sgemm_f32_")):
+        with _handle() as h:
+            run, check, _ = _split_product(h, False, 2048, 2048, 2048, call)
+            ib.check(run())
+            h.synchronize()
+            check()
+            assert name in h.last_implementation()
+            assert ("split3" in h.last_implementation()) == (h.scratch_usage()[0] > 0) == (call is ib.iclblasSgemm)
