@@ -19,16 +19,18 @@
 // FP32 MFMA, which rounds every fourth or second product, is at 3.1e-7 and 11.9e-7. The
 // additions run beside the MFMAs and cost 3% at 8192^3.
 //
-// What bounds it: at 8192^3 the card's power. The three-plane kernel runs at 1640
-// TFLOP/s of BF16 and 1.9 GHz (registers alone reach 2050 on random data),
-// so the choices here are those that cost least energy per product:
+// What bounds it: at 8192^3 the card's power. The three-plane kernel runs at 1570 to
+// 1640 TFLOP/s of BF16 (registers alone reach 2050 on random data), its matrix pipes busy
+// 83% of the cycles and the clock down to 1.75 to 1.9 GHz, where the FP32 MFMA kernel
+// holds 2.3: the choices here are those that cost least energy per product,
 // v_mfma_f32_16x16x32 (2048 TFLOP/s from registers against 1812 for 32x32x16), planes
 // kept in registers over as many groups of products as possible (36 LDS reads per 192
 // products; with the planes paired in 16-deep slabs, 56, it took 4.55 ms) and operands
 // copied to LDS without passing through registers. Four waves of 128 x 128 (a third fewer
 // LDS reads) do not fit the registers. SGEMM 8192^3: FP32 MFMA 7.75 ms, three planes
-// 4.29 ms, of which 0.27 the prepass (4.9 TB/s); CGEMM 4096^3 3.88 -> 2.16 ms. Two planes
-// 8192^3: 2.25 ms, against 2.52 with 32x32x16 MFMA and fragments read just before use.
+// 4.36 to 4.50 ms from card to card, of which 0.27 the prepass (4.9 TB/s); CGEMM 4096^3
+// 3.88 -> 2.2 to 2.3 ms. Two planes 8192^3: 2.25 to 2.35 ms, 1.11 to 1.13 times the rate
+// of 32x32x16 MFMA with fragments read just before use.
 // The 128 x 128 tile, two workgroups per CU, serves outputs with too few large tiles;
 // eight waves of 64 x 32, because a wave alone on its SIMD issues nothing beside its
 // MFMAs (2048^3: 84 us, with four of 64 x 64 101).
@@ -680,8 +682,8 @@ inline int sp_round_up(int x, int m) { return (x + m - 1) / m * m; }
 // 3.9 for a 256 x 256 tile, 2.15 for two 128 x 128 tiles on a CU and 1.25 for one (two
 // planes 2.05, 1.15, 0.65); 14 or 5 more per round of workgroups, which store C together
 // (4000 x 4000 x 512: 100 us with the large tile, 90 with the small); 4 and the
-// partial sums at 2.7 TB/s (written, and read again) for a split. SSYRK 640 (k 20011): 15 tiles in 34 parts, 745 -> 120 us; 1024 x
-// 1024 x 4096 139 -> 62 us.
+// partial sums at 2.7 TB/s (written, and read again) for a split. SSYRK 640 (k 20011):
+// 15 tiles in 34 parts, 745 -> 122 us; 1024 x 1024 x 4096 139 -> 62 us.
 // With a triangular operand (kband) the tiles start longest window first, so they fill
 // the CUs evenly and the longest is the bound: STRMM 3000 x 2048, all tiles in two
 // parts, 140 -> 95 us.

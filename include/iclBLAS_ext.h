@@ -15,12 +15,18 @@
  *    outside stream capture, on BF16 MFMA with every operand split exactly into
  *    three BF16 numbers (six products, FP32 accumulation): no bit of an operand
  *    is lost and the error is below FP32 MFMA's. Operands with elements that do
- *    not split exactly (infinities, NaN, magnitudes of 2^50 and more or below
- *    2^-110) take FP32 MFMA. ICLBLAS_MATH_SPLIT_BF16X3 splits every FP32 operand x into
- *    hi = bf16(x), lo = bf16(x - hi) and forms hi*hi + hi*lo + lo*hi on BF16
- *    MFMA with FP32 accumulation, for products at least 256 deep (shallower
- *    ones stay on FP32 MFMA); the error stays within the FP32 bound
- *    4 k 2^-24 (|A||B|).
+ *    not split exactly (infinities, NaN, magnitudes of 2^50 and more, or below
+ *    2^-110 and not 0) are found while they are packed, and the product then runs
+ *    on FP32 MFMA. On top of that such a call pays for what was packed until then
+ *    and an empty launch (8192^3 7.80 -> 7.83 ms, 2048^3 143 -> 161 us with 1 in
+ *    1000 elements out of range; up to 0.3 ms at 8192^3 for a single one), and
+ *    iclblasGetLastImplementation still names the kernel tried first. A call that
+ *    has to grow the workspace, 8 GiB at most, waits for the handle's stream and
+ *    allocates; under a scratch cap (iclblasSetScratchLimit) none does.
+ *    ICLBLAS_MATH_SPLIT_BF16X3 splits every FP32 operand x into hi = bf16(x),
+ *    lo = bf16(x - hi) and forms hi*hi + hi*lo + lo*hi on BF16 MFMA with FP32
+ *    accumulation, for products at least 256 deep (shallower ones run as in the
+ *    FP32 mode); the error stays within the FP32 bound 4 k 2^-24 (|A||B|).
  *  - Refined STRSM: FP32 blocked solve followed by sweeps of iterative
  *    refinement whose residual R = alpha*B - op(A)*X is formed in FP64.
  *  - Adjoints of SGEMM and STRSM.
@@ -134,9 +140,13 @@ ICLBLAS_API iclblasStatus_t iclblasGetKernelTiming(iclblasHandle_t handle, float
  * scratch that stages host matrices in the host-pointer mode and holds the
  * workspaces: packed split-BF16 operands, TRSM and refinement temporaries,
  * level-3 expansions, GEMV partial sums), in bytes; 0 (the default) removes
- * the cap. Under a cap the FP32 math mode keeps to kernels without workspaces. A call that would grow them beyond it returns
- * ICLBLAS_STATUS_ALLOC_FAILED, as when the device runs out of memory; buffers
- * already held are kept. Lowering the cap frees nothing. */
+ * the cap. Under a cap the FP32 math mode keeps to kernels without workspaces,
+ * and a split-BF16 product is refused only if its operands packed once do not
+ * fit (4 bytes per element, rows rounded up to tiles of 128 or 256; 8 complex).
+ * A call that would grow the buffers beyond the cap first gives up what only
+ * makes calls faster (packed operands of the FP32 mode) and else returns
+ * ICLBLAS_STATUS_ALLOC_FAILED, as when the device runs out of memory; the other
+ * buffers already held are kept. Lowering the cap frees nothing by itself. */
 ICLBLAS_API iclblasStatus_t iclblasSetScratchLimit(iclblasHandle_t handle, size_t bytes);
 /* Bytes the handle's buffers hold now, and the cap (0 = none). */
 ICLBLAS_API iclblasStatus_t iclblasGetScratchUsage(iclblasHandle_t handle, size_t* held, size_t* limit);
@@ -146,18 +156,19 @@ ICLBLAS_API iclblasStatus_t iclblasGetScratchUsage(iclblasHandle_t handle, size_
 
 /* SGEMM that allocates no memory. No counterpart in the reference: it is for
  * callers that cannot allocate (code under HIP graph capture, tight serving
- * loops, harnesses that forbid hipMalloc). Same arguments and validation
- * as iclblasSgemm and a result within the same error bound, except that A, B and C are always device pointers
- * (whatever the memory mode) and the call is queued on the handle's stream and
- * returns without waiting. It calls no hipMalloc, hipFree or other allocating
- * routine: in the split-BF16 math mode the packed operands go to a device
- * array of ICLBLAS_NOALLOC_SCRATCH_BYTES that the library holds on each GPU
- * from its first iclblasCreate there until the process ends. A call whose
- * packed operands need more than that, (M + N) * K * 4 bytes with M and N
- * rounded up to the kernel tile (256) and K to 32, returns
- * ICLBLAS_STATUS_INVALID_VALUE and queues nothing; the FP32 math mode (always on
- * FP32 MFMA here) and products shallower than 256 use no scratch and have no
- * such limit.
+ * loops, harnesses that forbid hipMalloc). Same arguments and validation as
+ * iclblasSgemm and a result within the same error bound (not always the same
+ * bits: iclblasSgemm may use memory that this call may not), except that A, B
+ * and C are always device pointers (whatever the memory mode) and the call is
+ * queued on the handle's stream and returns without waiting. It calls no
+ * hipMalloc, hipFree or other allocating routine: in the split-BF16 math mode
+ * the packed operands go to a device array of ICLBLAS_NOALLOC_SCRATCH_BYTES that
+ * the library holds on each GPU from its first iclblasCreate there until the
+ * process ends. A call whose packed operands need more than that, (M + N) * K * 4
+ * bytes with M and N rounded up to the kernel tile (128 or 256) and K to 32,
+ * returns ICLBLAS_STATUS_INVALID_VALUE and queues nothing; the FP32 math mode
+ * (always on FP32 MFMA here) and products shallower than 256 use no scratch and
+ * have no such limit.
  * ICLBLAS_STATUS_NOT_INITIALIZED: the scratch could not be set up on the
  * handle's GPU. Every call on one GPU shares that GPU's array: calls that
  * overlap on one GPU (other streams, other handles) race and must be ordered
