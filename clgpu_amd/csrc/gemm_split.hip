@@ -65,7 +65,7 @@ typedef __attribute__((address_space(3))) void sp_lds_void;
 // call's epoch into *guard, and the FP32 MFMA kernel computes the product instead. What
 // such a call pays on top of that kernel: the blocks packed until one of them finds an
 // element, and a launch that does nothing (1 in 1000 elements outside: 8192^3 7.80 ms of
-// FP32 MFMA -> 7.83, 4096^3 986 -> 1004 us, 2048^3 143 -> 161, 1500^3 138 -> 144).
+// FP32 MFMA -> 7.88, 4096^3 988 -> 1012 us, 2048^3 143 -> 162, 1500^3 138 -> 144).
 // ---------------------------------------------------------------------------
 struct SplitSrc {
     const float* X;
@@ -89,12 +89,15 @@ split_pack_kernel(SplitSrc a, SplitSrc b, int ablocks, int slabs, unsigned long 
 {
     __shared__ float T[64][64 + 1];
     const bool is_a = (int)blockIdx.x < ablocks;
-    const SplitSrc o = is_a ? a : b;
+    SplitSrc o = is_a ? a : b;
     const int r0 = (is_a ? (int)blockIdx.x : (int)blockIdx.x - ablocks) * 64; // packed row
     const int by = (int)(blockIdx.y + gridDim.y * blockIdx.z), k0 = by * 64;  // packed k
     if (2 * by >= slabs) return; // the last layer of a deep grid
-    // Nothing is packed any more once an element outside the range has been found.
-    if (PLANES == 3 && __hip_atomic_load(guard, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT) == epoch) return;
+    // Nothing is read or packed any more once an element outside the range has been found
+    // (waves may see that apart: all of them go through the barrier).
+    const bool off = PLANES == 3 && __builtin_amdgcn_readfirstlane(
+        __hip_atomic_load(guard, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT) == epoch);
+    if (off) o.R = 0;
     const int t = threadIdx.x;
     bool bad = false;
     if constexpr (!CPLX) {
@@ -141,11 +144,11 @@ split_pack_kernel(SplitSrc a, SplitSrc b, int ablocks, int slabs, unsigned long 
             }
         }
     }
-    if (PLANES == 3 && bad) *guard = epoch;
+    if (PLANES == 3 && bad) *guard = epoch; // (an atomic store of every such lane: 2048^3 161 -> 243 us)
     __syncthreads();
     // wave w writes k = 16 w .. 16 w + 15 of slab pair by, lane = row: 1 KB per store
     const int w = t >> 6, r = t & 63, ks = 2 * by + (w >> 1);
-    if (ks >= slabs) return;
+    if (off || ks >= slabs) return;
     bf16x8 out[PLANES][2];
 #pragma unroll
     for (int i = 0; i < 16; ++i) {

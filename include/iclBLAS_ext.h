@@ -18,7 +18,7 @@
  *    not split exactly (infinities, NaN, magnitudes of 2^50 and more, or below
  *    2^-110 and not 0) are found while they are packed, and the product then runs
  *    on FP32 MFMA. On top of that such a call pays for what was packed until then
- *    and an empty launch (8192^3 7.80 -> 7.83 ms, 2048^3 143 -> 161 us with 1 in
+ *    and an empty launch (8192^3 7.80 -> 7.88 ms, 2048^3 143 -> 162 us with 1 in
  *    1000 elements out of range; up to 0.3 ms at 8192^3 for a single one), and
  *    iclblasGetLastImplementation still names the kernel tried first. A call that
  *    has to grow the workspace, 8 GiB at most, waits for the handle's stream and
